@@ -3,6 +3,7 @@
 #pragma once
 
 #include "k_calc.h"
+#include "ldl_host.h"
 
 namespace fvh {
 
@@ -141,16 +142,21 @@ struct LevelStore {
 }  // namespace fvh
 
 namespace fvh {
-// LDL preconditioner: the factor of the set-up matrix in its ordering (L by
-// rows for the forward solve, by columns for the backward one), its pivots,
-// the solve's work vectors and a pinned fault word.
+// LDL preconditioner: the factor of the set-up matrix in its ordering (the
+// block solves' two sides, or, for the row solves, L by rows and by columns),
+// its pivots, the solves' work vectors and a pinned fault word.
+struct LdlSideDev {
+    DBuf<int> ptr, idx;
+    DBuf<double> val, inv;
+    DBuf<LdlBlock> blocks;
+    int nblocks = 0;
+};
 struct LdlStore {
     bool ready = false;
-    int nnzL = 0;
-    DBuf<int> perm, fptr, fidx, bptr, bidx;
-    DBuf<int> ranges;  // bounds of the nested-dissection leaves and separators (at most kLdlRangeMax rows each)
-    int nranges = 0;
-    DBuf<double> fval, bval, D, rhs, y, z;
+    bool by_blocks = true;
+    LdlSideDev f, b;  // row solves: ptr / idx / val alone
+    DBuf<int> perm;
+    DBuf<double> D, rhs, y, z, r, s;
     int *h_fault = nullptr;
     LdlStore() = default;
     LdlStore(const LdlStore &) = delete;

@@ -17,8 +17,12 @@
 #include "fvh_internal.h"
 
 #include <algorithm>
+#include <array>
+#include <atomic>
 #include <cmath>
 #include <numeric>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "ldl_host.h"
@@ -36,29 +40,33 @@ struct NdState {
     std::vector<int> *bounds;  // end of every leaf and separator appended (or null)
 };
 
-constexpr int kNdLeaf = 48;
+// Dissection goes on to kNdLeaf cells (less fill); a part of at most kNdRange
+// cells is one range, whose triangle one block inverts and applies: larger
+// ranges trade bytes (the packed inverse, s^2 / 2 values) for depth.
+constexpr int kNdLeaf = 48, kNdRange = kLdlLeaf;
 
 void nd_split(NdState &S, std::vector<int> cells) {
     // explicit stack instead of recursion: (cells, state) frames
     struct Frame {
         std::vector<int> cells;
         int stage;  // 0: split; 1: append separator after children
+        bool inside;  // part of a range whose end an enclosing frame marks
         std::vector<int> sep;
     };
     std::vector<Frame> st;
-    st.push_back({std::move(cells), 0, {}});
+    st.push_back({std::move(cells), 0, false, {}});
     while (!st.empty()) {
         Frame &F = st.back();
         if (F.stage == 1) {
             S.out->insert(S.out->end(), F.sep.begin(), F.sep.end());
-            if (S.bounds && !F.sep.empty()) S.bounds->push_back((int)S.out->size());
+            if (S.bounds && !F.inside && S.bounds->back() < (int)S.out->size()) S.bounds->push_back((int)S.out->size());
             st.pop_back();
             continue;
         }
         if ((int)F.cells.size() <= kNdLeaf) {
             std::sort(F.cells.begin(), F.cells.end());
             S.out->insert(S.out->end(), F.cells.begin(), F.cells.end());
-            if (S.bounds && !F.cells.empty()) S.bounds->push_back((int)S.out->size());
+            if (S.bounds && !F.inside && !F.cells.empty()) S.bounds->push_back((int)S.out->size());
             st.pop_back();
             continue;
         }
@@ -86,13 +94,15 @@ void nd_split(NdState &S, std::vector<int> cells) {
         }
         right.assign(v.begin() + half, v.end());
         std::sort(sep.begin(), sep.end());
+        // (a part small enough for one range is marked once, after its separator)
+        const bool inside = F.inside || (int)F.cells.size() <= kNdRange;
         F.stage = 1;
         F.sep = std::move(sep);
         F.cells.clear();
         F.cells.shrink_to_fit();
         // right is numbered after left: push it first (the stack pops left first)
-        st.push_back({std::move(right), 0, {}});
-        st.push_back({std::move(left), 0, {}});
+        st.push_back({std::move(right), 0, inside, {}});
+        st.push_back({std::move(left), 0, inside, {}});
     }
 }
 
@@ -150,6 +160,9 @@ int ldl_factor(int n, const int *rowptr, const int *col, const double *val, cons
     // numeric: row k of L from a sparse triangular solve along the etree
     std::vector<double> yv(n, 0.0);
     std::vector<int> pattern(n), fill(n, 0);
+    double *__restrict__ y = yv.data();
+    const int *__restrict__ Li = F.Li.data();
+    const double *__restrict__ Lx = F.Lx.data();
     for (int k = 0; k < n; ++k) {
         int top = n;
         flag[k] = k;
@@ -171,8 +184,8 @@ int ldl_factor(int n, const int *rowptr, const int *col, const double *val, cons
             const int i = pattern[top];
             const double yi = yv[i];
             yv[i] = 0.0;
-            const int p2 = F.Lp[i] + fill[i];
-            for (int p = F.Lp[i]; p < p2; ++p) yv[F.Li[p]] -= F.Lx[p] * yi;
+            const int p1 = F.Lp[i], p2 = p1 + fill[i];
+            for (int p = p1; p < p2; ++p) y[Li[p]] -= Lx[p] * yi;
             const double lki = yi / F.D[i];
             d -= lki * yi;
             F.Li[p2] = k;
@@ -184,6 +197,146 @@ int ldl_factor(int n, const int *rowptr, const int *col, const double *val, cons
         F.D[k] = d;
     }
     return FVH_OK;
+}
+
+// Inverse of the unit lower triangular block of s rows from r0, packed
+// without its unit diagonal by rows (row i: columns 0 .. i-1) and by columns
+// (column k: rows k+1 .. s-1), into the sides that read it so.  X: scratch.
+static void invert_range(const LdlHost &F, int r0, int s, std::vector<double> &X, bool whole, double *f, double *b) {
+    if (X.size() < (size_t)s * s) X.resize((size_t)s * s);
+    // X starts as the block itself (below its diagonal); row i of the inverse
+    // then replaces row i: -sum_k L_ik (row k of the inverse), k ascending (L_ik
+    // stands until its turn)
+    for (int i = 0; i < s; ++i) std::fill_n(&X[(size_t)i * s], i, 0.0);
+    for (int k = 0; k < s; ++k)
+        for (int p = F.Lp[r0 + k]; p < F.Lp[r0 + k + 1] && F.Li[p] < r0 + s; ++p)
+            X[(size_t)(F.Li[p] - r0) * s + k] = F.Lx[p];
+    for (int i = 1; i < s; ++i) {
+        double *xi = &X[(size_t)i * s];
+        for (int k = 0; k < i; ++k) {
+            const double l = xi[k];
+            if (l == 0.0) continue;
+            const double *xk = &X[(size_t)k * s];
+            for (int c = 0; c < k; ++c) xi[c] -= l * xk[c];
+            xi[k] = -l;
+        }
+    }
+    double *rows = whole ? b : f, *cols = whole ? f : b;  // a whole range: lane = row, column after column
+    for (int i = 1; i < s; ++i)
+        for (int k = 0; k < i; ++k) *rows++ = X[(size_t)i * s + k];
+    for (int k = 0; k + 1 < s; ++k)
+        for (int i = k + 1; i < s; ++i) *cols++ = X[(size_t)i * s + k];
+}
+
+void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out) {
+    const int n = F.n;
+    std::vector<int> cut{0};
+    for (size_t g = 0; g + 1 < bounds.size(); ++g)
+        for (int a = bounds[g]; a < bounds[g + 1]; a += kLdlRange) cut.push_back(std::min(a + kLdlRange, bounds[g + 1]));
+    const int ng = (int)cut.size() - 1;
+    std::vector<int> range_of(n);
+    for (int g = 0; g < ng; ++g)
+        for (int i = cut[g]; i < cut[g + 1]; ++i) range_of[i] = g;
+    // the entries outside the ranges' own blocks, by column and by row
+    LdlSide &f = out.f, &b = out.b;
+    f.ptr.assign(n + 1, 0);
+    b.ptr.assign(n + 1, 0);
+    for (int j = 0; j < n; ++j)
+        for (int p = F.Lp[j]; p < F.Lp[j + 1]; ++p)
+            if (range_of[F.Li[p]] != range_of[j]) {
+                f.ptr[F.Li[p] + 1]++;
+                b.ptr[j + 1]++;
+            }
+    for (int i = 0; i < n; ++i) {
+        f.ptr[i + 1] += f.ptr[i];
+        b.ptr[i + 1] += b.ptr[i];
+    }
+    f.idx.resize(f.ptr[n]);
+    f.val.resize(f.ptr[n]);
+    b.idx.resize(b.ptr[n]);
+    b.val.resize(b.ptr[n]);
+    // heights: a range follows, forward, every range its outside columns
+    // belong to, and backward every range its outside rows belong to
+    std::vector<int> hf(ng, 0), hb(ng, 0), pos(f.ptr.begin(), f.ptr.end() - 1);
+    for (int j = 0; j < n; ++j) {
+        const int g = range_of[j];
+        int q = b.ptr[j];
+        for (int p = F.Lp[j]; p < F.Lp[j + 1]; ++p) {
+            const int i = F.Li[p], gi = range_of[i];
+            if (gi == g) continue;
+            hf[gi] = std::max(hf[gi], hf[g] + 1);  // columns of g are all visited before those of gi
+            f.idx[pos[i]] = j;
+            f.val[pos[i]++] = F.Lx[p];
+            b.idx[q] = i;
+            b.val[q++] = F.Lx[p];
+        }
+    }
+    for (int j = n - 1; j >= 0; --j) {
+        const int g = range_of[j];
+        for (int p = b.ptr[j]; p < b.ptr[j + 1]; ++p) hb[g] = std::max(hb[g], hb[range_of[b.idx[p]]] + 1);
+    }
+    // inverse blocks, the ranges dealt to a few threads (each writes its own
+    // ranges' words)
+    std::vector<char> whole(ng);
+    std::vector<long long> off(ng + 1, 0);
+    for (int g = 0; g < ng; ++g) {
+        const long long s = cut[g + 1] - cut[g];
+        whole[g] = s <= kLdlWhole || (s <= kLdlLeaf && hf[g] == 0);
+        off[g + 1] = off[g] + s * (s - 1) / 2;
+    }
+    f.inv.resize(off[ng]);
+    b.inv.resize(off[ng]);
+    std::atomic<int> next{0};
+    const auto invert = [&] {
+        std::vector<double> X;
+        for (int g0; (g0 = next.fetch_add(64)) < ng;)
+            for (int g = g0; g < std::min(g0 + 64, ng); ++g)
+                invert_range(F, cut[g], cut[g + 1] - cut[g], X, whole[g], &f.inv[0] + off[g], &b.inv[0] + off[g]);
+    };
+    {
+        const int nt = off[ng] < (1 << 17) ? 1 : std::max(1, std::min(8, (int)std::thread::hardware_concurrency()));
+        std::vector<std::thread> th;
+        try {
+            for (int k = 1; k < nt; ++k) th.emplace_back(invert);
+        } catch (const std::system_error &) {  // fewer threads then
+        }
+        invert();
+        for (auto &t : th) t.join();
+    }
+    // a range's parent in the tree holds the first of its outside rows; a
+    // block's gates are words of the (at most two highest) ranges right below
+    // it (forward) or of the parent (backward)
+    std::vector<int> parent(ng, -1);
+    std::vector<std::array<int, 2>> child(ng, {-1, -1});
+    for (int g = 0; g < ng; ++g) {
+        int first = n;
+        for (int p = b.ptr[cut[g]]; p < b.ptr[cut[g + 1]]; ++p) first = std::min(first, b.idx[p]);
+        if (first == n) continue;
+        parent[g] = range_of[first];
+        std::array<int, 2> &c = child[parent[g]];
+        if (c[0] < 0 || hf[g] >= hf[c[0]]) c = {g, c[0]};
+        else if (c[1] < 0 || hf[g] > hf[c[1]]) c[1] = g;
+    }
+    const auto last_row = [&](int g) { return g < 0 ? -1 : cut[g + 1] - 1; };
+    // blocks by height (a range's outside rows before its inverse rows, which
+    // wait for the range's own last outside row)
+    const auto list = [&](const std::vector<int> &h, bool fwd, std::vector<LdlBlock> &blk) {
+        std::vector<int> order(ng);
+        std::iota(order.begin(), order.end(), 0);
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return h[x] < h[y]; });
+        for (int g : order) {
+            const int r0 = cut[g], s = cut[g + 1] - r0;
+            const int g0 = last_row(fwd ? child[g][0] : parent[g]), g1 = last_row(fwd ? child[g][1] : -1);
+            if (whole[g]) {
+                blk.push_back({0, r0, r0, s, {g0, g1}, off[g]});
+                continue;
+            }
+            for (int i = 0; i < s; i += kLdlWaves) blk.push_back({1, r0 + i, r0, s, {g0, g1}, off[g]});
+            for (int i = 0; i < s; i += kLdlWaves) blk.push_back({2, r0 + i, r0, s, {r0, r0 + s - 1}, off[g]});
+        }
+    };
+    list(hf, true, f.blocks);
+    list(hb, false, b.blocks);
 }
 
 }  // namespace fvh

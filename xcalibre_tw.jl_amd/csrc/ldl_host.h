@@ -23,4 +23,33 @@ void ldl_order(int n, const int *rowptr, const int *col, const double *x, const 
 // Numeric factorization; A symmetric (values read from its upper triangle).
 int ldl_factor(int n, const int *rowptr, const int *col, const double *val, const std::vector<int> &perm, LdlHost &F);
 
+// The factor as the block solves read it.  Per range of rows g the unit
+// lower triangular block L_gg is replaced by its explicit inverse, so that
+// the rows of a range do not wait for each other:
+//   forward   r_g = x_g - L_g,before y_before,        y_g = inv(L_gg) r_g
+//   backward  s_g = D_g^-1 y_g - L_after,g' z_after,  z_g = inv(L_gg)' s_g
+// Work is cut into blocks of kLdlWaves waves, listed in an order in which
+// every block follows the blocks whose results it reads.
+constexpr int kLdlWaves = 8;
+constexpr int kLdlWhole = 64;   // rows of a range that one block takes whole ...
+constexpr int kLdlLeaf = 80;    // ... and of a range without outside columns
+constexpr int kLdlRange = 512;  // rows of a range (longer ones are cut)
+struct LdlBlock {
+    int kind;           // 0: a whole range; 1: outside rows r, r+1, ... (a row per wave); 2: inverse rows
+    int r;              // first row
+    int r0, rows;       // its range
+    int gate[2];        // words its inputs are published with, last in the tree (-1: none)
+    long long off;      // the range's packed inverse
+};
+struct LdlSide {
+    std::vector<int> ptr, idx;  // per row (forward) or column (backward): the entries outside its range
+    std::vector<double> val, inv;
+    std::vector<LdlBlock> blocks;
+};
+struct LdlBlocks {
+    LdlSide f, b;
+};
+// `bounds`: ranges of positions in order (ldl_order's).
+void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out);
+
 }  // namespace fvh
