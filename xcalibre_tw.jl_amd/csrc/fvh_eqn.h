@@ -104,6 +104,7 @@ struct SkewStore {
     DBuf<double> uhand;
     SkewSweep<double> s64;
     SkewSweep<float> s32;
+    bool ilu = false;  // the records are ILU(0)'s
     int *h_fault = nullptr;
     SkewStore() = default;
     SkewStore(const SkewStore &) = delete;

@@ -33,6 +33,8 @@ struct SkewRect {
 int skew_setup(fvh_mesh *m, const std::vector<SkewRect> &rects);
 bool skew_active(const fvh_mesh *m);
 int skew_update(fvh_eqn *e, const double *val);
+// ILU(0) on the same sweeps (skew_apply and the FP32 and quad forms then apply it)
+int skew_ilu_update(fvh_eqn *e, const double *val);
 int skew_copy(fvh_eqn *e, const fvh_eqn *src);
 bool skew_tuned32(const fvh_mesh *m);  // the FP32 sweep width is chosen (tuned or forced)
 int skew_apply(fvh_eqn *e, const double *x, double *y, const KScal *ks);

@@ -40,7 +40,14 @@
 //   D_r   = (A_rr - (A_rs*A_sr)/D_s) - (A_rw*A_wr)/D_w,    Dinv_r = 1/D_r
 //   y_r   = (b_r - (A_rs*y_s)*Dinv_s) - (A_rw*y_w)*Dinv_w
 //   z_r   = (y_r*Dinv_r - (A_re*z_e)*Dinv_r) - (A_rn*z_n)*Dinv_r
-// and the results are bit-identical to the level-scheduled kernels for finite
+// ILU(0) runs the same pipeline (no fill of a five-point row meets the pattern
+// off its diagonal), with L = A / D formed beside D:
+//   D_r   = (A_rr - (A_rs/D_s)*A_sr) - (A_rw/D_w)*A_wr
+//   y_r   = (b_r - L_rs*y_s) - L_rw*y_w
+//   z_r   = ((y_r - A_re*z_e) - A_rn*z_n) / D_r
+// Its forward sweep is DILU's own with L for A and pivots of 1 (a product with
+// 1 is exact); its backward sweep divides, at the end of each step.
+// The results are bit-identical to the level-scheduled kernels for finite
 // data.  (A zero pivot or an infinite value can carry a NaN through a padding
 // slot into an edge cell where the reference has another non-finite value.)
 //
@@ -161,6 +168,9 @@ __device__ inline Rec4 bload(Rsrc r, unsigned vo, unsigned so, Rec4 *) {
     const auto u = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0));
     const auto v = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, vo + 16, so, 0));
     return Rec4{u.x, u.y, v.x, v.y};
+}
+__device__ inline double2 bload2(Rsrc r, unsigned vo, unsigned so) {
+    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0));
 }
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 __device__ inline void bstore(Rsrc r, double v, unsigned vo, unsigned so) {
@@ -404,7 +414,12 @@ struct Hand {
 // pass, all CUs, turns it into Dinv = 1/D afterwards, off the recurrence's
 // serial path)
 // ---------------------------------------------------------------------------
-template <int W>
+// ILU(0) (kIlu): U = (A_rr, A_nr, A_er, 0) and the coefficients (A_re, A_rn) of
+// Bk; each lane forms the terms its north and east neighbours subtract, with
+// those rows' own operands, (A_nr/D_r)*A_rn and (A_er/D_r)*A_re, right after
+// D_r: one division's latency between a step and the next instead of two rows'
+// pivots, and the cross-lane value is the finished term.
+template <int W, bool kIlu>
 __global__ void __launch_bounds__(64 * (W + 2))
     k_skew_update(SkewArgs a, const Rec4 *__restrict__ U, Rec4 *__restrict__ F, Rec4 *__restrict__ Bk,
                   double *__restrict__ hand) {
@@ -413,7 +428,7 @@ __global__ void __launch_bounds__(64 * (W + 2))
     const int b = blockIdx.x;
     const SkewGrid g = a.grids[a.blk_grid[b]];
     const int HS = a.HS, rb = b - g.blk0[W - 1], nb = (g.nw + W - 1) / W;
-    lds_reset(lds, (W + 1) * HS, HS, 1.0, rb == 0 ? 0 : -1);
+    lds_reset(lds, (W + 1) * HS, HS, kIlu ? 0.0 : 1.0, rb == 0 ? 0 : -1);
     __syncthreads();
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if (w == W) {  // incoming courier: D of the row below from block rb-1
@@ -437,20 +452,24 @@ __global__ void __launch_bounds__(64 * (W + 2))
     // the pre-start padding holds already, one record load), so that the
     // loop's memory waits count the same outstanding operations every step
     Rec4 ring[PD];
+    double2 re_rn[kIlu ? PD : 1];
     {
         const Rsrc ru = rsrc_at(U, a.rbytes, 0, step), rf = rsrc_at(F, a.rbytes, -PD, step);
+        const Rsrc rb2 = rsrc_at(Bk, a.rbytes, 0, step);
 #pragma unroll
         for (int k = 0; k < PD; ++k) {
             bstore(rf, 1.0, vo + 8, k * step);
             ring[k] = bload(ru, vo, k * step, (Rec4 *)nullptr);
+            if constexpr (kIlu) re_rn[k] = bload2(rb2, vo + 16, k * step);
             __builtin_amdgcn_sched_barrier(0);  // issue in consumption order
         }
     }
-    double dprev = 1.0, res[kL];
+    double dprev = kIlu ? 0.0 : 1.0, east = 0.0, res[kL];
     int broken = 0;
     int G0 = 0;
     do {
         // this iteration's steps G0*kL + i, i < kLook*kL: stores at i*step, refills PD steps on
+        const Rsrc rb2 = rsrc_at(Bk, a.rbytes, G0 * kL + PD, step);
         const Rsrc ru = rsrc_at(U, a.rbytes, G0 * kL + PD, step), rf = rsrc_at(F, a.rbytes, G0 * kL, step);
 #pragma unroll
         for (int h = 0; h < kLook; ++h) {
@@ -462,11 +481,20 @@ __global__ void __launch_bounds__(64 * (W + 2))
                 const unsigned si = (unsigned)(h * kL + k) * step;
                 const Rec4 u = ring[r];
                 const double ds = hd.template shift_in<true>(dprev, h, k);
-                const double d = (u.a - u.b / ds) - u.c / dprev;
+                double d;
+                if constexpr (kIlu) {  // dprev: the term for the row above
+                    d = (u.a - ds) - east;
+                    dprev = (u.b / d) * re_rn[r].y;
+                    east = (u.c / d) * re_rn[r].x;
+                } else {
+                    d = (u.a - u.b / ds) - u.c / dprev;
+                    dprev = d;
+                }
                 bstore(rf, d, vo + 8, si);
-                dprev = res[k] = d;
+                res[k] = dprev;
                 __builtin_amdgcn_sched_barrier(0);  // the slot is consumed: refill it below
                 ring[r] = bload(ru, vo, si, (Rec4 *)nullptr);
+                if constexpr (kIlu) re_rn[r] = bload2(rb2, vo + 16, si);
             }
             hd.finish(G, h, res);
         }
@@ -615,7 +643,8 @@ __global__ void __launch_bounds__(64 * (W + 2))
     if (broken) record_fault(a.fault);
 }
 
-template <typename T, int W>
+// kIlu (FP64 ILU(0)): quad records (D, A_re, A_rn)
+template <typename T, int W, bool kIlu>
 __global__ void __launch_bounds__(64 * (W + 2))
     k_skew_bwd(SkewArgs a, const T *__restrict__ kb, const T *__restrict__ yq, T *__restrict__ zp,
                T *__restrict__ hand, const KScal *ks) {
@@ -703,6 +732,9 @@ __global__ void __launch_bounds__(64 * (W + 2))
                     __builtin_amdgcn_sched_barrier(0);
                     const T zn = hd.template shift_in<false>(zprev, h, k);
                     z = __builtin_fmaf(-c[2], zn, t);
+                } else if constexpr (kIlu) {
+                    const T zn = hd.template shift_in<false>(zprev, h, k);
+                    z = ((y - c[1] * zprev) - c[2] * zn) / c[0];
                 } else {  // the reference's order of operations
                     const T zn = hd.template shift_in<false>(zprev, h, k);
                     z = ((y * c[0]) - c[1] * zprev * c[0]) - c[2] * zn * c[0];
@@ -742,13 +774,14 @@ __global__ void k_skew_fill(size_t ns, T *x, T v) {
 
 // Natural CSR values of the full-rectangle pattern -> skewed records; also
 // resets the diagonal recurrence's global hand-over arrays.
+template <bool kIlu>
 __global__ void k_skew_pack(int n, const SkewGrid *__restrict__ grids, const int *__restrict__ cell_grid,
                             const int *__restrict__ slot_of, const int *__restrict__ rowptr,
                             const int *__restrict__ diag, const double *__restrict__ val, Rec4 *__restrict__ F,
                             Rec4 *__restrict__ Bk, Rec4 *__restrict__ U, double *__restrict__ hand, int nhand,
                             int HS) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < nhand) hand[p] = (p % HS == 0) ? 1.0 : hand_sentinel<double>();
+    if (p < nhand) hand[p] = (p % HS == 0) ? (kIlu ? 0.0 : 1.0) : hand_sentinel<double>();
     if (p >= n) return;
     const SkewGrid g = grids[cell_grid ? cell_grid[p] : 0];
     const int rl = p - g.o, nx = g.nx;
@@ -761,7 +794,8 @@ __global__ void k_skew_pack(int n, const SkewGrid *__restrict__ grids, const int
     const double a_rw = Wn ? val[d - 1] : 0.0;                  // A[r, r-1]
     const double a_wr = Wn ? val[diag[p - 1] + 1] : 0.0;        // A[r-1, r]
     const int s = slot_of[p];
-    U[s] = Rec4{val[d], a_rs * a_sr, a_rw * a_wr, 0.0};
+    if constexpr (kIlu) U[s] = Rec4{val[d], a_nr, E ? val[diag[p + 1] - 1] : 0.0, 0.0};  // A[r+1, r]
+    else U[s] = Rec4{val[d], a_rs * a_sr, a_rw * a_wr, 0.0};
     F[s].c = a_nr;
     F[s].d = a_rw;
     Bk[s].c = E ? val[d + 1] : 0.0;                // A[r, r+1]
@@ -921,6 +955,37 @@ __global__ void k_skew_quads(const SkewGrid *__restrict__ grids, Rec4 *__restric
     for (int t = 0; t < 4 * NB; ++t) kb[NB * o + t] = cb[t];
 }
 
+// ILU(0) after its recurrence (D in F.b): L_nr = A_nr / D_r and L_rw = A_rw /
+// D_w into F (the division the factorization makes of the row's entry), 1 / D
+// into Bk.b (the FP32 quads) and (D, A_re, A_rn) into the backward quads.  F.b
+// is only read here (a row's west pivot is another thread's): the next kernel
+// sets it to the forward sweep's pivot, 1.
+__global__ void k_skew_ilu(const SkewGrid *__restrict__ grids, Rec4 *__restrict__ F, Rec4 *__restrict__ Bk,
+                           double *__restrict__ kb) {
+    const SkewGrid g = grids[blockIdx.y];
+    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= ((size_t)g.NG * kSkewL + 2 * kSkewPD) / 4 * g.S) return;
+    const int qi = (int)(q / g.S) + (kSkewQ0 - kSkewPD) / 4, j = (int)(q % g.S);
+    const size_t s0 = g.base + (size_t)(4 * qi - kSkewQ0 + kSkewD0) * g.S + j;  // slot of (T, j), word 0
+    const size_t o = g.base + (size_t)qi * 4 * g.S + 4 * (size_t)j;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const size_t s = s0 + (size_t)w * g.S;
+        const double d = F[s].b, dw = F[s - g.S].b;
+        const Rec4 v = Bk[s];
+        F[s].c = F[s].c / d;
+        F[s].d = F[s].d / dw;
+        Bk[s].b = 1.0 / d;
+        kb[kBwdN * (o + w)] = d;
+        kb[kBwdN * (o + w) + 1] = v.c;
+        kb[kBwdN * (o + w) + 2] = v.d;
+    }
+}
+__global__ void k_skew_unit_pivots(size_t ns, Rec4 *F) {
+    const size_t s = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < ns) F[s].b = 1.0;
+}
+
 __global__ void k_skew_dinv_natural(int n, const int *__restrict__ slot_of, const Rec4 *__restrict__ F,
                                     double *__restrict__ out) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1069,15 +1134,19 @@ static int sweep_alloc(SkewSweep<T> &w, const SkewLayout &L) {
     return FVH_OK;
 }
 
+static size_t most_quads(const SkewLayout &L) {
+    size_t most = 0;
+    for (const SkewGrid &g : L.h_grids) most = std::max(most, ((size_t)g.NG * kSkewL + 2 * kSkewPD) / 4 * g.S);
+    return most;
+}
+
 // The quad records of one precision from the current F and Bk.
 template <typename T>
 static int sweep_records(fvh_eqn *e, SkewSweep<T> &w) {
     const SkewLayout &L = *e->m->skew;
     FVH_TRY(sweep_alloc(w, L));
-    size_t most = 0;
-    for (const SkewGrid &g : L.h_grids) most = std::max(most, ((size_t)g.NG * kSkewL + 2 * kSkewPD) / 4 * g.S);
-    hipLaunchKernelGGL((k_skew_quads<T>), dim3((unsigned)((most + 255) / 256), (unsigned)L.h_grids.size()), dim3(256),
-                       0, stream(), L.grids.p, e->sk.F.p, e->sk.Bk.p, w.kf.p, w.kb.p);
+    hipLaunchKernelGGL((k_skew_quads<T>), dim3((unsigned)((most_quads(L) + 255) / 256), (unsigned)L.h_grids.size()),
+                       dim3(256), 0, stream(), L.grids.p, e->sk.F.p, e->sk.Bk.p, w.kf.p, w.kb.p);
     HIP_TRY(hipGetLastError());
     return FVH_OK;
 }
@@ -1098,12 +1167,12 @@ static int allow_lds(K kernel, size_t bytes) {
     return FVH_OK;
 }
 
-template <int W>
+template <int W, bool kIlu>
 static int launch_update_w(fvh_eqn *e) {
     const SkewLayout &L = *e->m->skew;
     const size_t lds = (size_t)(W + 1) * L.HS * sizeof(double);
-    FVH_TRY(allow_lds(k_skew_update<W>, lds));
-    hipLaunchKernelGGL((k_skew_update<W>), dim3(L.nblk[W - 1]), dim3(64 * (W + 2)), lds, stream(),
+    FVH_TRY(allow_lds(k_skew_update<W, kIlu>, lds));
+    hipLaunchKernelGGL((k_skew_update<W, kIlu>), dim3(L.nblk[W - 1]), dim3(64 * (W + 2)), lds, stream(),
                        skew_args<Rec4>(e, W), e->sk.U.p, e->sk.F.p, e->sk.Bk.p, e->sk.uhand.p);
     HIP_TRY(hipGetLastError());
     return FVH_OK;
@@ -1111,20 +1180,29 @@ static int launch_update_w(fvh_eqn *e) {
 
 static int skew_tune(fvh_eqn *e);
 
-int skew_update(fvh_eqn *e, const double *val) {
+// Records and diagonal recurrence from the natural values.
+template <bool kIlu>
+static int skew_factor(fvh_eqn *e, const double *val) {
     fvh_mesh *m = e->m;
     const SkewLayout &L = *m->skew;
     FVH_TRY(skew_alloc(e));
+    e->sk.ilu = kIlu;
     const int n = (int)m->n, nhand = L.nblk[0] * L.HS;
-    hipLaunchKernelGGL(k_skew_pack, grid_for(std::max(n, nhand)), dim3(256), 0, stream(), n, L.grids.p, cell_grid(m),
-                       L.slot_of.p, m->d.rowptr, m->d.diag, val, e->sk.F.p, e->sk.Bk.p, e->sk.U.p, e->sk.uhand.p,
-                       nhand, L.HS);
+    hipLaunchKernelGGL((k_skew_pack<kIlu>), grid_for(std::max(n, nhand)), dim3(256), 0, stream(), n, L.grids.p,
+                       cell_grid(m), L.slot_of.p, m->d.rowptr, m->d.diag, val, e->sk.F.p, e->sk.Bk.p, e->sk.U.p,
+                       e->sk.uhand.p, nhand, L.HS);
     HIP_TRY(hipGetLastError());
     switch (skew_waves(L)) {
-        case 1: FVH_TRY(launch_update_w<1>(e)); break;
-        case 2: FVH_TRY(launch_update_w<2>(e)); break;
-        default: FVH_TRY(launch_update_w<3>(e)); break;
+        case 1: return launch_update_w<1, kIlu>(e);
+        case 2: return launch_update_w<2, kIlu>(e);
+        default: return launch_update_w<3, kIlu>(e);
     }
+}
+
+int skew_update(fvh_eqn *e, const double *val) {
+    fvh_mesh *m = e->m;
+    const SkewLayout &L = *m->skew;
+    FVH_TRY(skew_factor<false>(e, val));
     int edge = 0;
     for (const SkewGrid &g : L.h_grids) edge = std::max(edge, g.nx + g.ny);
     hipLaunchKernelGGL(k_skew_edges, dim3((unsigned)((edge + 255) / 256), (unsigned)L.h_grids.size()), dim3(256), 0,
@@ -1132,6 +1210,19 @@ int skew_update(fvh_eqn *e, const double *val) {
     HIP_TRY(hipGetLastError());
     FVH_TRY(sweep_records(e, e->sk.s64));
     if (!m->skew->W && !forced_waves()) FVH_TRY(skew_tune(e));
+    return FVH_OK;
+}
+
+int skew_ilu_update(fvh_eqn *e, const double *val) {
+    const SkewLayout &L = *e->m->skew;
+    FVH_TRY(skew_factor<true>(e, val));
+    FVH_TRY(sweep_alloc(e->sk.s64, L));
+    hipLaunchKernelGGL(k_skew_ilu, dim3((unsigned)((most_quads(L) + 255) / 256), (unsigned)L.h_grids.size()), dim3(256),
+                       0, stream(), L.grids.p, e->sk.F.p, e->sk.Bk.p, e->sk.s64.kb.p);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_skew_unit_pivots, grid_for(L.NS), dim3(256), 0, stream(), L.NS, e->sk.F.p);
+    HIP_TRY(hipGetLastError());
+    if (!e->m->skew->W && !forced_waves()) FVH_TRY(skew_tune(e));
     return FVH_OK;
 }
 
@@ -1153,21 +1244,30 @@ int skew_copy(fvh_eqn *e, const fvh_eqn *src) {
     return FVH_OK;
 }
 
-template <typename T, int W>
+template <typename T, int W, bool kIlu>
 static int launch_sweeps_w(fvh_eqn *e, SkewSweep<T> &w, const KScal *ks) {
     const SkewLayout &L = *e->m->skew;
     const SkewArgs a = skew_args<Rec4T<T>>(e, W);
     const size_t lds = (size_t)(W + 1) * L.HS * sizeof(T), lds_f = lds;
     FVH_TRY(allow_lds(k_skew_fwd<T, W>, lds_f));
-    FVH_TRY(allow_lds(k_skew_bwd<T, W>, lds));
+    FVH_TRY(allow_lds(k_skew_bwd<T, W, kIlu>, lds));
     const void *recs = sizeof(T) == 8 ? static_cast<const void *>(e->sk.F.p) : w.kf.p;
     hipLaunchKernelGGL((k_skew_fwd<T, W>), dim3(a.nblk), dim3(64 * (W + 2)), lds_f, stream(), a, recs, w.bq.p, w.yq.p,
                        w.hand.p, ks);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL((k_skew_bwd<T, W>), dim3(a.nblk), dim3(64 * (W + 2)), lds, stream(), a, w.kb.p, w.yq.p, w.zp.p,
+    hipLaunchKernelGGL((k_skew_bwd<T, W, kIlu>), dim3(a.nblk), dim3(64 * (W + 2)), lds, stream(), a, w.kb.p, w.yq.p, w.zp.p,
                        w.hand.p, ks);
     HIP_TRY(hipGetLastError());
     return FVH_OK;
+}
+
+// FP32 ILU(0) applies the premultiplied records as DILU does
+template <typename T, int W>
+static int launch_sweeps_k(fvh_eqn *e, SkewSweep<T> &w, const KScal *ks) {
+    if constexpr (sizeof(T) == 8) {
+        if (e->sk.ilu) return launch_sweeps_w<T, W, true>(e, w, ks);
+    }
+    return launch_sweeps_w<T, W, false>(e, w, ks);
 }
 
 // gather with the reset of the hand-over arrays (skipped when the caller has
@@ -1190,9 +1290,9 @@ static int skew_sweeps_t(fvh_eqn *e, const T *x, const KScal *ks, SkewSweep<T> &
         HIP_TRY(hipGetLastError());
     }
     switch (skew_waves(L, sizeof(T) == 4)) {
-        case 1: FVH_TRY((launch_sweeps_w<T, 1>(e, w, ks))); break;
-        case 2: FVH_TRY((launch_sweeps_w<T, 2>(e, w, ks))); break;
-        default: FVH_TRY((launch_sweeps_w<T, 3>(e, w, ks))); break;
+        case 1: FVH_TRY((launch_sweeps_k<T, 1>(e, w, ks))); break;
+        case 2: FVH_TRY((launch_sweeps_k<T, 2>(e, w, ks))); break;
+        default: FVH_TRY((launch_sweeps_k<T, 3>(e, w, ks))); break;
     }
     return FVH_OK;
 }

@@ -183,6 +183,11 @@ static int ilu_setup(fvh_mesh *m) {
     return FVH_OK;
 }
 
+// ILU(0) runs on the pipelined band sweeps on a single full rectangle (250 x
+// 125: 65 us an apply, against 771 us on the one-work-group level walk, which
+// keeps the other meshes).
+static bool ilu_skew(const fvh_mesh *m) { return !m->cases && band_path(m) && skew_active(m); }
+
 int precond_update(fvh_eqn *eq) {
     fvh_eqn *e = eq->pshare ? eq->pshare : eq;  // preconditioner object (may be shared)
     fvh_mesh *m = e->m;
@@ -203,7 +208,11 @@ int precond_update(fvh_eqn *eq) {
             if (band_path(m)) return band_dilu_update(e, src->nz.p);
             if (lev_path(m)) return lev_dilu_update(e, src->nz.p);
             return dilu_update(m, src->nz.p, e->D.p, e->Dinv.p);
-        case FVH_PRECOND_ILU0: return ilu0_factor(m, src->nz.p, e->lu.p);
+        case FVH_PRECOND_ILU0:
+            if (ilu_skew(m)) return skew_ilu_update(e, src->nz.p);
+            FVH_TRY(ilu_setup(m));
+            if (e->lu.n != (size_t)m->nnz) FVH_TRY(e->lu.alloc(m->nnz));
+            return ilu0_factor(m, src->nz.p, e->lu.p);
         case FVH_PRECOND_LDL: return ldl_setup(e, src->nz.p);  // the first update factors; later ones keep it
         default: return set_error(FVH_ERR_UNSUPPORTED, "preconditioner %d", e->pkind);
     }
@@ -231,7 +240,10 @@ int precond_apply(fvh_eqn *eq, double *y, const double *x, const KScal *ks_in, d
             if (band_path(m)) return band_dilu_apply(e, x, y, ks_in);
             if (lev_path(m) && e->lv.fwd.p) return lev_dilu_apply(e, x, y, ks);
             return dilu_apply(m, src->nz.p, e->Dinv.p, x, y, ks);
-        case FVH_PRECOND_ILU0: return ilu0_apply(m, e->lu.p, x, y, ks);
+        case FVH_PRECOND_ILU0:
+            if (ilu_skew(m)) return skew_apply(e, x, y, ks_in);
+            if (!e->lu.p) return set_error(FVH_ERR_ARG, "ILU(0) preconditioner applied before its update");
+            return ilu0_apply(m, e->lu.p, x, y, ks);
         case FVH_PRECOND_LDL: return ldl_apply<double>(e, x, y, ks);
         default: return set_error(FVH_ERR_UNSUPPORTED, "preconditioner %d", e->pkind);
     }
@@ -318,6 +330,8 @@ int prepare32(fvh_eqn *e) {
             });
         }
         case FVH_PRECOND_ILU0: {
+            if (ilu_skew(m)) return skew_to32(P);
+            if (!P->lu.p) return set_error(FVH_ERR_ARG, "ILU(0) preconditioner applied before its update");
             if (P->p32b.n != (size_t)nnz) FVH_TRY(P->p32b.alloc(nnz));
             const double *lu = P->lu.p;
             float *lf = P->p32b.p;
@@ -344,7 +358,9 @@ int precond_apply32(fvh_eqn *eq, float *y, const float *x, const KScal *ks_in) {
             if (band_path(m)) return band_dilu_apply32(e, x, y, ks_in);
             if (lev_path(m) && e->lv.fwd32.p) return lev_dilu_apply32(e, x, y, ks);
             return dilu_apply32(m, e->p32b.p, e->p32a.p, x, y, ks);
-        case FVH_PRECOND_ILU0: return ilu0_apply32(m, e->p32b.p, x, y, ks);
+        case FVH_PRECOND_ILU0:
+            if (ilu_skew(m)) return skew_apply32(e, x, y, ks_in);
+            return ilu0_apply32(m, e->p32b.p, x, y, ks);
         case FVH_PRECOND_LDL: return ldl_apply<float>(e, x, y, ks);  // the FP64 factor, FP32 vectors
         default: return set_error(FVH_ERR_UNSUPPORTED, "preconditioner %d", e->pkind);
     }
@@ -457,14 +473,15 @@ static int sys_precond(const Sys<double> &S, double *y, const double *x, const K
 static int sys_precond(const Sys<float> &S, float *y, const float *x, const KScal *ks) {
     return precond_apply32(S.e, y, x, ks);
 }
-// The map of natural rows into the banded DILU sweeps' result quads when the
-// system's preconditioner is that apply (pipelined band sweeps, one case),
+// The map of natural rows into the banded DILU / ILU(0) sweeps' result quads
+// when the system's preconditioner is that apply (pipelined band sweeps, one case),
 // else null: CG then reads z from the quads and skips the scatter.
 template <typename T>
 static const int *sys_quad_map(const Sys<T> &S) {
     const fvh_eqn *P = S.e->pshare ? S.e->pshare : S.e;
     const fvh_mesh *m = S.e->m;
-    if (P->pkind != FVH_PRECOND_DILU || m->cases || !band_path(m) || !skew_active(m)) return nullptr;
+    if ((P->pkind != FVH_PRECOND_DILU && P->pkind != FVH_PRECOND_ILU0) || m->cases || !band_path(m) || !skew_active(m))
+        return nullptr;
     return skew_quad_map(m);
 }
 static int sys_precond_quads(const Sys<double> &S, const double *x, const KScal *ks, const double **zq) {
@@ -1303,8 +1320,10 @@ extern "C" int fvh_precond_set(fvh_eqn *e, int32_t kind, fvh_eqn *matrix_of) {
             FVH_TRY(e->Dinv.alloc(n));
             break;
         case FVH_PRECOND_ILU0:
-            FVH_TRY(ilu_setup(e->m));
-            FVH_TRY(e->lu.alloc(e->m->nnz));
+            if (!ilu_skew(e->m)) {
+                FVH_TRY(ilu_setup(e->m));
+                FVH_TRY(e->lu.alloc(e->m->nnz));
+            }
             break;
         case FVH_PRECOND_LDL:
             if (e->m->cases) return set_error(FVH_ERR_UNSUPPORTED, "LDL preconditioner: not with independent cases");
