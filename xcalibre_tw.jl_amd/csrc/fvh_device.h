@@ -92,8 +92,7 @@ struct DevMesh {
     const int *cf_ptr, *cf_face, *cf_nbr, *cf_slot;  // cell -> internal faces (faces_range order)
     const double *cf_sign, *cf_w, *cf_omw;           // nsign, divergence weights of that side
     int nif;                                         // internal faces (faces nbf .. nf-1)
-    const int2 *fi_slot;                             // internal face: slots of A[o, n] and A[n, o] (~slot: nsign -1)
-    const double2 *fi_w;                             // internal face: divergence weights of the o and n sides
+    const int *cf_fs;                                // cf_face with the side's nsign: f, or ~f when it is -1
     const int *own1, *own2;                          // face owners (boundary: own1 == own2)
     const double *fw, *farea, *fdelta;               // face weight, area, delta
     const double *Sfx, *Sfy, *Sfz;                   // area * normal
@@ -103,12 +102,15 @@ struct DevMesh {
     const double *ccx, *ccy, *ccz, *fcx, *fcy, *fcz;  // centres
     const int *cb_ptr, *cb_face;                     // cell -> boundary faces, ascending face id
     const int *bf_face, *bf_cell, *bf_patch;         // boundary faces in boundary (patch) order
+    const int *fb_patch;                             // the patch of boundary face f (-1: of none; its cell is own1)
 };
 
 // Per-cell boundary-condition entries of one BC tuple, in the order
 // apply_boundary_conditions! visits them (tuple order, then patch order).
 struct BcPlan {
     DBuf<int> ptr, face, bc;
+    DBuf<int> cells;  // the cells with entries, ascending
+    int ncells = 0;
 };
 
 // Anti-diagonal geometry of a banded grid, by value in kernel arguments.
@@ -261,12 +263,9 @@ struct fvh_mesh {
     int nboundaries = 0;
     // owned device storage
     fvh::DBuf<int> rowptr, col, diag, tslot, cf_ptr, cf_face, cf_nbr, cf_slot, own1, own2, cb_ptr, cb_face,
-        bf_face, bf_cell, bf_patch, fi_slot;
-    fvh::DBuf<double> fi_w, ex, ey, ez;
+        bf_face, bf_cell, bf_patch, cf_fs, fb_patch;
+    fvh::DBuf<double> ex, ey, ez;
     bool cf_ascending = true;  // every cell's internal faces in ascending face id
-    // per-slot diagonal terms handed from the face pass of the assembly to
-    // its cell pass ([slot][face term]); sized by the largest term count seen
-    fvh::DBuf<double> asm_terms;
     fvh::DBuf<double> cf_sign, cf_w, cf_omw, fw, farea, fdelta, Sfx, Sfy, Sfz, nx, ny, nz, vol, ccx, ccy, ccz, fcx,
         fcy, fcz;
     // host copies used by set-up code

@@ -23,14 +23,18 @@ struct AsmArgs {
     int mode;
     int nterms;
     KTerm t[kMaxTerms];
-    int nft;              // face terms (Laplacian, Divergence), set by launch_assemble
-    KTerm ft[kMaxTerms];  // ... in model order
+    // set by launch_assemble: the face terms (Laplacian, Divergence) in model
+    // order, and whether a Laplacian / a linear divergence is among them
+    int nft, laplacian, linear_div;
+    KTerm ft[kMaxTerms];
     int nsrc;
     double ssign[kMaxSrc];
     const double *sfield[kMaxSrc];
     const double *prev;  // Time{Euler} previous values (null = 0)
     double rdt;
     const int *bptr, *bface, *bbc;  // fused boundary conditions (null = none)
+    const int *bcells;              // the cells that have some (ASM_BC_ONLY)
+    int nbcells;
     BcVals bc;
     int relax;
     double alpha;

@@ -1,18 +1,20 @@
 // Discretise: face-loop assembly of the model terms into A (CSR values) and
 // b, with boundary conditions, implicit relaxation and the pressure
-// reference fused into the cell pass.
+// reference fused in.
 //
-// Two passes, no atomics.  The face pass (one thread per internal face,
-// face arrays read coalesced) evaluates every face term for the owner and
-// the neighbour side (Discretise_1_schemes.jl:40-92), writes the two
-// off-diagonal slots through the precomputed face->CSR slot map, and leaves
-// each side's diagonal terms in a per-slot array.  The cell pass (one
-// thread per cell) sums those terms in the reference's order
+// One pass, one thread per cell, no atomics: a cell writes its own row, taking
+// its faces four at a time.  It evaluates every face term for its side
+// (Discretise_1_schemes.jl:40-92) in the reference's order
 // (Discretise_2_generated_distretisation.jl:55-73):
 //   faces in faces_range order (terms in model order)
 //   -> scheme_source! terms -> sources
 //   -> boundary conditions (BC tuple order, then patch face order, then terms)
 //   -> implicit relaxation -> setReference!.
+// Bound by HBM.  Each face is read by both its cells, the second time mostly
+// from a cache (its cells are near each other), and its coefficient is formed
+// twice.  That moves 56 % of the bytes of a face pass that hands each side's
+// diagonal terms to a cell pass through memory (2000 x 1000 quads, two face
+// terms: 178 us; this pass: 101 us).
 #include "fvh_eqn.h"
 
 namespace fvh {
@@ -54,96 +56,75 @@ __device__ inline void apply_bc_entries(const DevMesh &m, const AsmArgs &a, int 
     }
 }
 
-// Face pass: one thread per internal face, reading the face arrays
-// coalesced.  It evaluates every face term for both sides of the face
-// (owner o with its nsign, neighbour n with its own), writes the two
-// off-diagonal slots A[o, n] and A[n, o] (each the sum of its terms from 0
-// in model order, as the reference accumulates them into the zeroed
-// nzval), and hands the per-side diagonal terms to the cell pass through
-// td[slot][term], indexed by the off-diagonal slot of that side.
+// NFT >= 0: the rows of cells 0 .. count-1 from their faces, then the cell
+// terms and sources; NFT < 0: the diagonal and b of cells list[0 .. count-1]
+// (null: first + 0 .. count-1) as they stand.  Then boundary conditions,
+// implicit relaxation and the reference cell.  A row's off-diagonal entry is
+// the sum of its face's terms from 0 in model order, as the reference
+// accumulates them into the zeroed nzval; the diagonal is summed term by term
+// over the faces.
 template <int NFT>
-__global__ void __launch_bounds__(256) k_asm_faces(DevMesh m, AsmArgs a, double *__restrict__ nz,
-                                                   double *__restrict__ td) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m.nif) return;
-    const int f = m.nbf + k;
-    const int2 sv = m.fi_slot[k];
-    const int so = sv.x >= 0 ? sv.x : ~sv.x, sn = sv.y >= 0 ? sv.y : ~sv.y;
-    const double nso = sv.x >= 0 ? 1.0 : -1.0, nsn = sv.y >= 0 ? 1.0 : -1.0;
-    double offo = 0.0, offn = 0.0;
-    double dto[NFT > 0 ? NFT : 1], dtn[NFT > 0 ? NFT : 1];
-#pragma unroll
-    for (int q = 0; q < NFT; ++q) {
-        const KTerm &t = a.ft[q];
-        const double flux = t.flux[f];
-        if (t.op == FVH_OP_LAPLACIAN) {
-            // the same coefficient on both sides (no nsign)
-            const double ap = (t.sign * (-flux * m.farea[f])) / m.fdelta[f];
-            dto[q] = ap;
-            dtn[q] = ap;
-            offo += -ap;
-            offn += -ap;
-        } else {
-            const double apo = t.sign * (flux * nso), apn = t.sign * (flux * nsn);
-            if (t.scheme == FVH_LINEAR) {
-                const double2 w = m.fi_w[k];
-                dto[q] = apo * (1.0 - w.x);
-                dtn[q] = apn * (1.0 - w.y);
-                offo += apo * w.x;
-                offn += apn * w.y;
-            } else {
-                dto[q] = jmax0(apo);
-                dtn[q] = jmax0(apn);
-                offo += -jmax0(-apo);
-                offn += -jmax0(-apn);
-            }
-        }
-    }
-    nz[so] = offo;
-    nz[sn] = offn;
-#pragma unroll
-    for (int q = 0; q < NFT; ++q) {
-        td[(size_t)so * NFT + q] = dto[q];
-        td[(size_t)sn * NFT + q] = dtn[q];
-    }
-}
-
-// Cell pass: one thread per cell.  NFT >= 0: full assembly, the diagonal
-// summed from 0 over the cell's internal faces in faces_range order, terms
-// in model order within a face (the face pass's per-side terms), then the
-// cell terms and sources; NFT < 0: the diagonal and b as they stand.  Then
-// boundary conditions, implicit relaxation and the reference cell.
-template <int NFT>
-__global__ void __launch_bounds__(256) k_asm_cells(DevMesh m, AsmArgs a, const double *__restrict__ td,
-                                                   double *__restrict__ nz, double *__restrict__ bv) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= m.n) return;
+__global__ void __launch_bounds__(256) k_asm_cells(DevMesh m, AsmArgs a, int count, const int *__restrict__ list,
+                                                   int first, double *__restrict__ nz, double *__restrict__ bv) {
+    const int q0 = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q0 >= count) return;
+    const int c = NFT >= 0 ? q0 : (list ? list[q0] : first + q0);
     const int dslot = m.diag[c];
     double diag, b;
     if (NFT >= 0) {
         diag = 0.0;
         if (NFT > 0) {
-            // four sides at a time: their slot loads, then their terms'
-            // loads, issued together; summed in faces_range order
+            // four sides at a time: their index loads, then their faces'
+            // loads, issued together
             constexpr int G = 4, NT = NFT > 0 ? NFT : 1;
             const int i1 = m.cf_ptr[c + 1];
             for (int i = m.cf_ptr[c]; i < i1; i += G) {
-                int sl[G];
-                double v[G][NT];
-#pragma unroll
-                for (int k = 0; k < G; ++k)
-                    if (i + k < i1) sl[k] = m.cf_slot[i + k];
+                int fs[G], sl[G];
+                double v[G][NT], ar[G], de[G], w[G];
 #pragma unroll
                 for (int k = 0; k < G; ++k)
                     if (i + k < i1) {
-#pragma unroll
-                        for (int q = 0; q < NT; ++q) v[k][q] = td[(size_t)sl[k] * NT + q];
+                        fs[k] = m.cf_fs[i + k];
+                        sl[k] = m.cf_slot[i + k];
                     }
 #pragma unroll
                 for (int k = 0; k < G; ++k)
                     if (i + k < i1) {
+                        const int f = fs[k] >= 0 ? fs[k] : ~fs[k];
 #pragma unroll
-                        for (int q = 0; q < NT; ++q) diag += v[k][q];
+                        for (int q = 0; q < NT; ++q) v[k][q] = a.ft[q].flux[f];
+                        if (a.laplacian) {
+                            ar[k] = m.farea[f];
+                            de[k] = m.fdelta[f];
+                        }
+                        if (a.linear_div) w[k] = m.cf_w[i + k];
+                    }
+#pragma unroll
+                for (int k = 0; k < G; ++k)
+                    if (i + k < i1) {
+                        const double ns = fs[k] >= 0 ? 1.0 : -1.0;
+                        double off = 0.0;
+#pragma unroll
+                        for (int q = 0; q < NT; ++q) {
+                            const KTerm &t = a.ft[q];
+                            const double flux = v[k][q];
+                            if (t.op == FVH_OP_LAPLACIAN) {
+                                // the same coefficient on both sides (no nsign)
+                                const double ap = (t.sign * (-flux * ar[k])) / de[k];
+                                diag += ap;
+                                off += -ap;
+                            } else {
+                                const double ap = t.sign * (flux * ns);
+                                if (t.scheme == FVH_LINEAR) {
+                                    diag += ap * (1.0 - w[k]);
+                                    off += ap * w[k];
+                                } else {
+                                    diag += jmax0(ap);
+                                    off += -jmax0(-ap);
+                                }
+                            }
+                        }
+                        nz[sl[k]] = off;
                     }
             }
         }
@@ -231,42 +212,39 @@ int check_bc_terms(const AsmArgs &a, const fvh_bc *bcs, int nbc) {
 }
 
 template <int NFT>
-static int launch_full(fvh_eqn *e, const AsmArgs &a) {
-    fvh_mesh *m = e->m;
-    double *td = nullptr;
-    if (NFT > 0) {
-        const size_t need = (size_t)m->nnz * NFT;
-        if (m->asm_terms.n < need) FVH_TRY(m->asm_terms.alloc(need));
-        td = m->asm_terms.p;
-    }
-    if (m->d.nif > 0) {
-        hipLaunchKernelGGL((k_asm_faces<NFT>), grid1d(m->d.nif), dim3(256), 0, stream(), m->d, a, e->nz.p, td);
-        HIP_TRY(hipGetLastError());
-    }
-    hipLaunchKernelGGL((k_asm_cells<NFT>), grid1d(m->n), dim3(256), 0, stream(), m->d, a, td, e->nz.p, e->b.p);
+static int launch_cells(fvh_eqn *e, const AsmArgs &a, int count, const int *list, int first) {
+    if (count <= 0) return FVH_OK;
+    hipLaunchKernelGGL((k_asm_cells<NFT>), grid1d(count), dim3(256), 0, stream(), e->m->d, a, count, list, first,
+                       e->nz.p, e->b.p);
     HIP_TRY(hipGetLastError());
     return FVH_OK;
 }
 
-// Full assembly: the face pass then the cell pass (the face terms compacted
-// into a.ft in model order); the partial modes run the cell pass alone.
+// Full assembly (the face terms compacted into a.ft in model order); the
+// partial modes visit only the cells they change: boundary conditions the
+// cells of the plan, a reference value its cell.
 int launch_assemble(fvh_eqn *e, const AsmArgs &a0) {
+    const int n = (int)e->m->n;
+    if (a0.mode == ASM_BC_ONLY && a0.bcells) return launch_cells<-1>(e, a0, a0.nbcells, a0.bcells, 0);
     if (a0.mode != ASM_FULL) {
-        hipLaunchKernelGGL((k_asm_cells<-1>), grid1d(e->m->n), dim3(256), 0, stream(), e->m->d, a0, nullptr, e->nz.p,
-                           e->b.p);
-        HIP_TRY(hipGetLastError());
-        return FVH_OK;
+        if (a0.setref && !a0.refflag && !a0.relax && !a0.bptr) return launch_cells<-1>(e, a0, 1, nullptr, a0.refcell);
+        return launch_cells<-1>(e, a0, n, nullptr, 0);
     }
     AsmArgs a = a0;
     a.nft = 0;
+    a.laplacian = a.linear_div = 0;
     for (int i = 0; i < a.nterms; ++i)
-        if (a.t[i].op == FVH_OP_LAPLACIAN || a.t[i].op == FVH_OP_DIVERGENCE) a.ft[a.nft++] = a.t[i];
+        if (a.t[i].op == FVH_OP_LAPLACIAN || a.t[i].op == FVH_OP_DIVERGENCE) {
+            a.ft[a.nft++] = a.t[i];
+            if (a.t[i].op == FVH_OP_LAPLACIAN) a.laplacian = 1;
+            else if (a.t[i].scheme == FVH_LINEAR) a.linear_div = 1;
+        }
     switch (a.nft) {
-        case 0: return launch_full<0>(e, a);
-        case 1: return launch_full<1>(e, a);
-        case 2: return launch_full<2>(e, a);
-        case 3: return launch_full<3>(e, a);
-        case 4: return launch_full<4>(e, a);
+        case 0: return launch_cells<0>(e, a, n, nullptr, 0);
+        case 1: return launch_cells<1>(e, a, n, nullptr, 0);
+        case 2: return launch_cells<2>(e, a, n, nullptr, 0);
+        case 3: return launch_cells<3>(e, a, n, nullptr, 0);
+        case 4: return launch_cells<4>(e, a, n, nullptr, 0);
         default: return set_error(FVH_ERR_SIZE, "at most %d face terms", kMaxTerms);
     }
 }
@@ -339,6 +317,8 @@ extern "C" int fvh_apply_bcs(fvh_eqn *e, const fvh_term *terms, int32_t nterms, 
     a.bptr = plan->ptr.p;
     a.bface = plan->face.p;
     a.bbc = plan->bc.p;
+    a.bcells = plan->cells.p;
+    a.nbcells = plan->ncells;
     FVH_TRY(launch_assemble(e, a));
     HIP_TRY(hipStreamSynchronize(stream()));
     return FVH_OK;

@@ -26,11 +26,32 @@ __global__ void k_interpolate_vec(DevMesh m, const double *__restrict__ ux, cons
     fy[f] = w * uy[c1] + omw * uy[c2];
 }
 
-// interpolate_midpoint! for scalars: 0.5*(phi1 + phi2) on all faces
-__global__ void k_interpolate_midpoint(DevMesh m, const double *__restrict__ phi, double *__restrict__ phif) {
-    int f = blockIdx.x * blockDim.x + threadIdx.x;
+// interpolate! (or, MID, interpolate_midpoint!: 0.5*(phi1 + phi2)) and
+// correct_boundaries! in one launch: a boundary face that a BC names takes the
+// corrected value (k_correct_boundaries below), every other face the
+// interpolated one.  500 k triangles: 8.0 + 3.4 us in two launches, 8.1 us
+// in one.
+template <bool MID>
+__global__ void k_interpolate_bc(DevMesh m, BcVals bc, const double *__restrict__ phi, double *__restrict__ phif) {
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= m.nf) return;
-    phif[f] = 0.5 * (phi[m.own1[f]] + phi[m.own2[f]]);
+    if (f < m.nbf) {
+        const int patch = m.fb_patch[f];
+        int hit = -1;
+        for (int k = 0; k < bc.nbc; ++k)
+            if (bc.patch[k] == patch) hit = k;
+        if (hit >= 0) {
+            phif[f] = (bc.kind[hit] == FVH_BC_DIRICHLET) ? bc.value[hit] : phi[m.own1[f]];
+            return;
+        }
+    }
+    const double p1 = phi[m.own1[f]], p2 = phi[m.own2[f]];
+    if constexpr (MID) {
+        phif[f] = 0.5 * (p1 + p2);
+    } else {
+        const double w = m.fw[f], omw = 1.0 - w;
+        phif[f] = w * p1 + omw * p2;
+    }
 }
 
 // interpolate_midpoint! for vectors: weight*(x1 + x2) (Calculate_0_gradient.jl:140)
@@ -96,8 +117,9 @@ __global__ void k_green_gauss(DevMesh m, const double *__restrict__ phif, double
 #pragma unroll
         for (int k = 0; k < kFaceGroup; ++k)
             if (i + k < i1) {
-                f[k] = m.cf_face[i + k];
-                ns[k] = m.cf_sign[i + k];
+                const int fs = m.cf_fs[i + k];
+                f[k] = fs >= 0 ? fs : ~fs;
+                ns[k] = fs >= 0 ? 1.0 : -1.0;
             }
 #pragma unroll
         for (int k = 0; k < kFaceGroup; ++k)
@@ -161,8 +183,9 @@ __global__ void k_div(DevMesh m, const double *__restrict__ fx, const double *__
 #pragma unroll
         for (int k = 0; k < kFaceGroup; ++k)
             if (i + k < i1) {
-                f[k] = m.cf_face[i + k];
-                ns[k] = m.cf_sign[i + k];
+                const int fs = m.cf_fs[i + k];
+                f[k] = fs >= 0 ? fs : ~fs;
+                ns[k] = fs >= 0 ? 1.0 : -1.0;
             }
 #pragma unroll
         for (int k = 0; k < kFaceGroup; ++k)
@@ -362,9 +385,8 @@ int launch_nonorthogonal_correct(const fvh_mesh *m, int sign, const double *J, c
 int launch_grad(const fvh_mesh *m, int scheme, const BcVals &bc, const double *phi, double *phif, double *dx, double *dy,
                 double *dz) {
     if (scheme == FVH_MIDPOINT) {
-        hipLaunchKernelGGL(k_interpolate_midpoint, grid_of(m->nf), dim3(256), 0, stream(), m->d, phi, phif);
+        hipLaunchKernelGGL((k_interpolate_bc<true>), grid_of(m->nf), dim3(256), 0, stream(), m->d, bc, phi, phif);
         HIP_TRY(hipGetLastError());
-        FVH_TRY(launch_correct_boundaries(m, bc, phi, phif));
         FVH_TRY(launch_green_gauss(m, phif, dx, dy, dz));
         for (int it = 0; it < 2; ++it) {
             FVH_TRY(launch_correct_interpolation(m, dx, dy, dz, phi, phif));
@@ -373,8 +395,8 @@ int launch_grad(const fvh_mesh *m, int scheme, const BcVals &bc, const double *p
         return FVH_OK;
     }
     if (scheme != FVH_ORTHOGONAL) return set_error(FVH_ERR_UNSUPPORTED, "gradient scheme %d", scheme);
-    FVH_TRY(launch_interpolate(m, phi, phif));
-    FVH_TRY(launch_correct_boundaries(m, bc, phi, phif));
+    hipLaunchKernelGGL((k_interpolate_bc<false>), grid_of(m->nf), dim3(256), 0, stream(), m->d, bc, phi, phif);
+    HIP_TRY(hipGetLastError());
     return launch_green_gauss(m, phif, dx, dy, dz);
 }
 

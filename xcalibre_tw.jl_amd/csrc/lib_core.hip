@@ -72,8 +72,9 @@ int bc_plan(fvh_mesh *m, const fvh_bc *bcs, int nbc, BcPlan **out) {
         int b = bcs[k].patch;
         for (int i = m->h_bstart[b]; i < m->h_bstart[b + 1]; ++i) per[m->h_bf_cell[i]].push_back({m->h_bf_face[i], k});
     }
-    std::vector<int> ptr(n + 1, 0), face, bc;
+    std::vector<int> ptr(n + 1, 0), face, bc, cells;
     for (int c = 0; c < n; ++c) {
+        if (!per[c].empty()) cells.push_back(c);
         for (auto &e : per[c]) {
             face.push_back(e.first);
             bc.push_back(e.second);
@@ -84,6 +85,8 @@ int bc_plan(fvh_mesh *m, const fvh_bc *bcs, int nbc, BcPlan **out) {
     FVH_TRY(plan->ptr.upload(ptr));
     FVH_TRY(plan->face.upload(face));
     FVH_TRY(plan->bc.upload(bc));
+    FVH_TRY(plan->cells.upload(cells));
+    plan->ncells = (int)cells.size();
     *out = plan.get();
     m->bc_plans.emplace(key, std::move(plan));
     return FVH_OK;
@@ -430,12 +433,11 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
             cf_w[i] = w;
             cf_omw[i] = 1.0 - w;
         }
-    // internal faces seen from the face: the slots A[o, n] and A[n, o] and
-    // the two sides' divergence weights, for the face-parallel assembly pass
+    // every internal face is listed once by each of its two owners; the side's
+    // nsign rides in the face's sign bit: ~face when -1
     const int nif = nf - nbf;
-    constexpr int kNoSide = INT32_MIN;
-    std::vector<int> fi_slot(2 * (size_t)std::max(nif, 1), kNoSide);
-    std::vector<double> fi_w(2 * (size_t)std::max(nif, 1), 0.0);
+    std::vector<int> cf_fs(ncf);
+    std::vector<char> listed(2 * (size_t)std::max(nif, 1), 0);
     for (int c = 0; c < n; ++c)
         for (int i = cf_ptr[c]; i < cf_ptr[c + 1]; ++i) {
             const int f = cf_face[i];
@@ -443,13 +445,12 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
             const int side = (own1[f] == c) ? 0 : (own2[f] == c ? 1 : -1);
             if (side < 0) return set_error(FVH_ERR_MESH, "cell %d lists face %d of which it is no owner", c, f);
             const size_t k = 2 * (size_t)(f - nbf) + side;
-            if (fi_slot[k] != kNoSide) return set_error(FVH_ERR_MESH, "face %d listed twice by cell %d", f, c);
-            // the side's nsign rides in the slot's sign bit: ~slot when -1
-            fi_slot[k] = cf_sign[i] > 0.0 ? cf_slot[i] : ~cf_slot[i];
-            fi_w[k] = cf_w[i];
+            if (listed[k]) return set_error(FVH_ERR_MESH, "face %d listed twice by cell %d", f, c);
+            listed[k] = 1;
+            cf_fs[i] = cf_sign[i] > 0.0 ? f : ~f;
         }
     for (int k = 0; k < 2 * nif; ++k)
-        if (fi_slot[k] == kNoSide) return set_error(FVH_ERR_MESH, "internal face %d is missing from a cell's face list", nbf + k / 2);
+        if (!listed[k]) return set_error(FVH_ERR_MESH, "internal face %d is missing from a cell's face list", nbf + k / 2);
     // cell -> boundary faces in ascending face id
     std::vector<int> cb_ptr(n + 1, 0), cb_face;
     for (int f = 0; f < nbf; ++f) cb_ptr[own1[f] + 1]++;
@@ -505,8 +506,7 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
     FVH_TRY(m->cf_sign.upload(cf_sign));
     FVH_TRY(m->cf_w.upload(cf_w));
     FVH_TRY(m->cf_omw.upload(cf_omw));
-    FVH_TRY(m->fi_slot.upload(fi_slot));
-    FVH_TRY(m->fi_w.upload(fi_w));
+    FVH_TRY(m->cf_fs.upload(cf_fs));
     FVH_TRY(m->own1.upload(own1));
     FVH_TRY(m->own2.upload(own2));
     FVH_TRY(m->cb_ptr.upload(cb_ptr));
@@ -514,6 +514,9 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
     FVH_TRY(m->bf_face.upload(bf_face));
     FVH_TRY(m->bf_cell.upload(bf_cell));
     FVH_TRY(m->bf_patch.upload(bf_patch));
+    std::vector<int> fb_patch(nbf, -1);
+    for (int i = 0; i < nbf; ++i) fb_patch[bf_face[i]] = bf_patch[i];
+    FVH_TRY(m->fb_patch.upload(fb_patch));
     FVH_TRY(m->fw.upload(fw));
     FVH_TRY(m->farea.upload(farea));
     FVH_TRY(m->fdelta.upload(fdelta));
@@ -552,12 +555,13 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
     v.rowptr = m->rowptr.p; v.col = m->col.p; v.diag = m->diag.p; v.tslot = m->tslot.p;
     v.cf_ptr = m->cf_ptr.p; v.cf_face = m->cf_face.p; v.cf_nbr = m->cf_nbr.p; v.cf_slot = m->cf_slot.p;
     v.cf_sign = m->cf_sign.p; v.cf_w = m->cf_w.p; v.cf_omw = m->cf_omw.p;
-    v.nif = nif; v.fi_slot = (const int2 *)m->fi_slot.p; v.fi_w = (const double2 *)m->fi_w.p;
+    v.nif = nif; v.cf_fs = m->cf_fs.p;
     v.own1 = m->own1.p; v.own2 = m->own2.p; v.fw = m->fw.p; v.farea = m->farea.p; v.fdelta = m->fdelta.p;
     v.Sfx = m->Sfx.p; v.Sfy = m->Sfy.p; v.Sfz = m->Sfz.p; v.nx = m->nx.p; v.ny = m->ny.p; v.nz = m->nz.p;
     v.ex = m->ex.p; v.ey = m->ey.p; v.ez = m->ez.p;
     v.vol = m->vol.p; v.ccx = m->ccx.p; v.ccy = m->ccy.p; v.ccz = m->ccz.p; v.fcx = m->fcx.p; v.fcy = m->fcy.p; v.fcz = m->fcz.p;
     v.cb_ptr = m->cb_ptr.p; v.cb_face = m->cb_face.p;
+    v.fb_patch = m->fb_patch.p;
     v.bf_face = m->bf_face.p; v.bf_cell = m->bf_cell.p; v.bf_patch = m->bf_patch.p;
     *out = m.release();
     return FVH_OK;
