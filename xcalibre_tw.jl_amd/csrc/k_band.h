@@ -62,6 +62,12 @@ int skew_rhs_target(fvh_eqn *e, int fp32, SkewRhs *t);
 // the reset of the hand-over arrays alone (the gather's other half)
 int skew_hand_reset(fvh_eqn *e, int fp32);
 int skew_dinv_natural(fvh_eqn *e, double *out);
+// CG iterations of a small grid in one launch: whether the mesh's do, and up
+// to `steps` of them (band: A by band position)
+bool skew_cg_fits(const fvh_mesh *m, int fp32);
+template <typename T>
+int skew_cg_small(fvh_eqn *e, const T *band, T *x, T *r, T *z, T *p, T *Ap, double sigma, double epsT, int steps,
+                  int itmax, KScal *ks);
 // reports (once) a sweep whose hand-over wait ran out
 int skew_check(fvh_eqn *e);
 

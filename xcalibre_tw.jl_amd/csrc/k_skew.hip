@@ -60,6 +60,7 @@
 #include "fvh_eqn.h"
 #include "k_band.h"
 #include "k_dpp.h"
+#include "k_spmv.h"
 
 namespace fvh {
 
@@ -528,31 +529,14 @@ __global__ void __launch_bounds__(64 * (W + 2))
 constexpr int kFwdN = 2;  // FP32 forward quad records
 constexpr int kBwdN = 3;
 
-template <typename T, int W>
-__global__ void __launch_bounds__(64 * (W + 2))
-    k_skew_fwd(SkewArgs a, const void *__restrict__ recs, const T *__restrict__ bq, T *__restrict__ yq,
-               T *__restrict__ hand, const KScal *ks) {
+// One compute wave of the forward sweep: wave wg of the grid (rows 64 wg + lane),
+// reading the hand-over array `lin` and writing `lout`.
+template <typename T>
+__device__ __forceinline__ void fwd_wave(const SkewArgs &a, const SkewGrid &g, int wg, const T *lin, T *lout,
+                                         const void *__restrict__ recs, const T *__restrict__ bq,
+                                         T *__restrict__ yq) {
     using R = Rec4T<T>;
-    extern __shared__ unsigned char skew_lds[];
-    T *lds = reinterpret_cast<T *>(skew_lds);
-    const int b = blockIdx.x;
-    const int gi = a.blk_grid[b];
-    if (ks && ks[a.ks_per_grid ? gi : 0].done) return;
-    const SkewGrid g = a.grids[gi];
-    const int HS = a.HS, rb = b - g.blk0[W - 1], nb = (g.nw + W - 1) / W;
-    lds_reset(lds, (W + 1) * HS, HS, T(0), rb == 0 ? 0 : -1);
-    __syncthreads();
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (w == W) {  // couriers: the forward channel of block b is hand[2b]
-        courier_in(rb > 0 ? hand + (size_t)(b - 1) * 2 * HS : nullptr, lds, g.NG, a.fault);
-        return;
-    }
-    if (w == W + 1) {
-        courier_out(lds + W * HS, rb < nb - 1 ? hand + (size_t)b * 2 * HS : nullptr, g.NG, a.fault);
-        return;
-    }
-    if (rb * W + w >= g.nw) return;  // past the grid's last wave (last block)
-    const int lane = threadIdx.x & 63, wg = rb * W + w;
+    const int HS = a.HS, lane = threadIdx.x & 63;
     const unsigned S = g.S, j0 = wg * 64;
     const unsigned vo = (g.base + j0 + lane) * (unsigned)sizeof(R), step = S * (unsigned)sizeof(R);
     // lane q < kL of the batch of group G holds step G*kL + q
@@ -566,7 +550,7 @@ __global__ void __launch_bounds__(64 * (W + 2))
     const unsigned vc = N * vq, cstride = N * step;
     const R *F = static_cast<const R *>(recs);
     Hand<T> hd;
-    hd.start(lds + w * HS, lds + (w + 1) * HS, HS, ql, lane == 63, g.NG);
+    hd.start(lin, lout, HS, ql, lane == 63, g.NG);
     R ring[kFused ? 1 : PD];           // FP64 records
     Vec<T, 4 * N> cr[kFused ? NR : 1];  // FP32 coefficient quads
     Vec<T, 4> br[kFused ? NR : 1];      // FP32 right-hand-side quads
@@ -643,33 +627,38 @@ __global__ void __launch_bounds__(64 * (W + 2))
     if (broken) record_fault(a.fault);
 }
 
-// kIlu (FP64 ILU(0)): quad records (D, A_re, A_rn)
-template <typename T, int W, bool kIlu>
+template <typename T, int W>
 __global__ void __launch_bounds__(64 * (W + 2))
-    k_skew_bwd(SkewArgs a, const T *__restrict__ kb, const T *__restrict__ yq, T *__restrict__ zp,
+    k_skew_fwd(SkewArgs a, const void *__restrict__ recs, const T *__restrict__ bq, T *__restrict__ yq,
                T *__restrict__ hand, const KScal *ks) {
-    using R = Rec4T<T>;
     extern __shared__ unsigned char skew_lds[];
     T *lds = reinterpret_cast<T *>(skew_lds);
-    const int b = a.nblk - 1 - (int)blockIdx.x;  // top row blocks first
+    const int b = blockIdx.x;
     const int gi = a.blk_grid[b];
     if (ks && ks[a.ks_per_grid ? gi : 0].done) return;
     const SkewGrid g = a.grids[gi];
     const int HS = a.HS, rb = b - g.blk0[W - 1], nb = (g.nw + W - 1) / W;
-    // the grid's top wave reads the array above it, which nobody writes
-    lds_reset(lds, (W + 1) * HS, HS, T(0), rb == nb - 1 ? g.nw - rb * W : -1);
+    lds_reset(lds, (W + 1) * HS, HS, T(0), rb == 0 ? 0 : -1);
     __syncthreads();
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (w == W) {  // couriers: the backward channel of block b is hand[2b+1]
-        courier_in(rb < nb - 1 ? hand + ((size_t)(b + 1) * 2 + 1) * HS : nullptr, lds + W * HS, g.NG, a.fault);
+    if (w == W) {  // couriers: the forward channel of block b is hand[2b]
+        courier_in(rb > 0 ? hand + (size_t)(b - 1) * 2 * HS : nullptr, lds, g.NG, a.fault);
         return;
     }
     if (w == W + 1) {
-        courier_out(lds, rb > 0 ? hand + ((size_t)b * 2 + 1) * HS : nullptr, g.NG, a.fault);
+        courier_out(lds + W * HS, rb < nb - 1 ? hand + (size_t)b * 2 * HS : nullptr, g.NG, a.fault);
         return;
     }
     if (rb * W + w >= g.nw) return;  // past the grid's last wave (last block)
-    const int lane = threadIdx.x & 63, wg = rb * W + w;
+    fwd_wave<T>(a, g, rb * W + w, lds + w * HS, lds + (w + 1) * HS, recs, bq, yq);
+}
+
+// One compute wave of the backward sweep.  kIlu (FP64 ILU(0)): quad records (D, A_re, A_rn)
+template <typename T, bool kIlu>
+__device__ __forceinline__ void bwd_wave(const SkewArgs &a, const SkewGrid &g, int wg, const T *lin, T *lout,
+                                         const T *__restrict__ kb, const T *__restrict__ yq, T *__restrict__ zp) {
+    using R = Rec4T<T>;
+    const int HS = a.HS, lane = threadIdx.x & 63;
     const unsigned S = g.S, j0 = wg * 64;
     const int Ttop = g.NG * kL - 1;  // step u handles anti-diagonal Ttop - u
     const unsigned step = S * (unsigned)sizeof(R);  // bytes per quad of values
@@ -680,7 +669,7 @@ __global__ void __launch_bounds__(64 * (W + 2))
     constexpr int M = ring_batches<T>(), PD = M * kL;
     static_assert(kLook % M == 0, "whole rings per unrolled block");
     Hand<T> hd;
-    hd.start(lds + (w + 1) * HS, lds + w * HS, HS, qh, lane == 0, g.NG);
+    hd.start(lin, lout, HS, qh, lane == 0, g.NG);
     // Ttop + 1 + kSkewQ0 is a multiple of 4, so step i of an iteration is
     // word 3 - i%4 of the iteration's quad i/4 (four diagonals, descending)
     constexpr bool kFused = sizeof(T) == 4;
@@ -753,6 +742,33 @@ __global__ void __launch_bounds__(64 * (W + 2))
         G0 += kLook;
     } while (G0 < g.NG);
     if (broken) record_fault(a.fault);
+}
+
+template <typename T, int W, bool kIlu>
+__global__ void __launch_bounds__(64 * (W + 2))
+    k_skew_bwd(SkewArgs a, const T *__restrict__ kb, const T *__restrict__ yq, T *__restrict__ zp,
+               T *__restrict__ hand, const KScal *ks) {
+    extern __shared__ unsigned char skew_lds[];
+    T *lds = reinterpret_cast<T *>(skew_lds);
+    const int b = a.nblk - 1 - (int)blockIdx.x;  // top row blocks first
+    const int gi = a.blk_grid[b];
+    if (ks && ks[a.ks_per_grid ? gi : 0].done) return;
+    const SkewGrid g = a.grids[gi];
+    const int HS = a.HS, rb = b - g.blk0[W - 1], nb = (g.nw + W - 1) / W;
+    // the grid's top wave reads the array above it, which nobody writes
+    lds_reset(lds, (W + 1) * HS, HS, T(0), rb == nb - 1 ? g.nw - rb * W : -1);
+    __syncthreads();
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (w == W) {  // couriers: the backward channel of block b is hand[2b+1]
+        courier_in(rb < nb - 1 ? hand + ((size_t)(b + 1) * 2 + 1) * HS : nullptr, lds + W * HS, g.NG, a.fault);
+        return;
+    }
+    if (w == W + 1) {
+        courier_out(lds, rb > 0 ? hand + ((size_t)b * 2 + 1) * HS : nullptr, g.NG, a.fault);
+        return;
+    }
+    if (rb * W + w >= g.nw) return;  // past the grid's last wave (last block)
+    bwd_wave<T, kIlu>(a, g, rb * W + w, lds + (w + 1) * HS, lds + w * HS, kb, yq, zp);
 }
 
 // ---------------------------------------------------------------------------
@@ -990,6 +1006,196 @@ __global__ void k_skew_dinv_natural(int n, const int *__restrict__ slot_of, cons
                                     double *__restrict__ out) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p < n) out[p] = F[slot_of[p]].b;
+}
+
+// ---------------------------------------------------------------------------
+// CG iterations of a small grid in one work-group (see skew_cg_small)
+// ---------------------------------------------------------------------------
+constexpr int kCgThreads = 256;     // one wave per SIMD: two would leave the sweeps 128 VGPRs (they need 193)
+constexpr int kCgMaxChunks = 2;
+static_assert(kCgThreads == kBlock, "thread = lane of the canonical reduction");
+
+// Rows of a chunk in groups of kPer per thread: all a group's loads (load(i))
+// are in flight before the first of its results (use(i, v)) is formed.  Rows
+// past n re-read the last one and are dropped.
+template <class Load, class Use>
+__device__ inline void block_rows(int n, int c, Load load, Use use) {
+    decltype(load(0)) v[kPer];
+    const int i0 = c * kChunk + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) v[k] = load(min(i0 + k * kCgThreads, n - 1));
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) use(i0 + k * kCgThreads, v[k]);
+}
+
+// Canonical sum over rows of term(i, load(i)), from every thread of the block:
+// chunk by chunk as chunk_reduce forms the partials (lane t adds rows t +
+// 256 k in order), then as final_reduce adds at most kCgMaxChunks of them
+// (lane t of its tree holds partial t, and the lanes beyond are zeros).
+template <class Load, class Term>
+__device__ inline double block_sum(int n, int nch, double *sp, double *part, Load load, Term term) {
+    const int t = threadIdx.x;
+    for (int c = 0; c < nch; ++c) {
+        double acc = 0.0;
+        block_rows(n, c, load, [&](int i, const decltype(load(0)) &v) {
+            if (i < n) acc = acc + term(i, v);
+        });
+        sp[t] = acc;
+        __syncthreads();
+        if (t < 128) sp[t] = sp[t] + sp[t + 128];
+        __syncthreads();
+        if (t < 64) {
+            double v = sp[t] + sp[t + 64];
+            v = v + __shfl_down(v, 32);
+            v = v + __shfl_down(v, 16);
+            v = v + __shfl_down(v, 8);
+            v = v + __shfl_down(v, 4);
+            v = v + __shfl_down(v, 2);
+            v = v + __shfl_down(v, 1);
+            if (t == 0) part[c] = v;
+        }
+        __syncthreads();
+    }
+    static_assert(kCgMaxChunks == 2, "the tree's last level");
+    return (0.0 + part[0]) + (nch > 1 ? 0.0 + part[1] : 0.0);
+}
+
+template <typename T>
+struct CgSmall {
+    SkewArgs a;
+    int n, nch, nx, steps, itmax, stride;
+    const unsigned char *mask;
+    const T *C;                     // A by band position
+    T sg;                           // sigma as the SpMV applies it ...
+    double sigma, epsT;             // ... and as the recurrence does
+    T *x, *r, *z, *p, *Ap, *bdst;   // bdst[map[i] * stride]: the forward sweep's right-hand side
+    const int *map, *qmap;
+    const void *recs;
+    T *bq, *yq, *zp;
+    const T *kb;
+    KScal *ks;
+};
+
+// Up to `steps` CG iterations, expression for expression and sum for sum those
+// of cg() (k_solve.hip) with its kernels (k_cg_alpha, k_cg_beta,
+// k_spmv_dot_band, k_mapred), so the bits are the same.  p holds the next
+// iteration's direction at the end of each one.
+template <typename T, bool kIlu>
+__global__ void __launch_bounds__(kCgThreads) k_cg_small(CgSmall<T> s) {
+    extern __shared__ unsigned char skew_lds[];
+    __shared__ double sp[kCgThreads], part[kCgMaxChunks];
+    KScal *ks = s.ks;
+    if (ks->done) return;
+    const SkewGrid g = s.a.grids[0];
+    const int HS = s.a.HS, nw = g.nw, t = threadIdx.x, n = s.n, half = (nw + 1) * HS;
+    T *fl = reinterpret_cast<T *>(skew_lds), *bl = fl + half;  // hand-over arrays of the two sweeps
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    double gamma = ks->gamma, pn2 = ks->pnorm2, gprev = ks->gprev, alpha = ks->alpha, beta = ks->beta,
+           rnorm = ks->rnorm;
+    const double eps = ks->eps;
+    int iter = ks->iter, done = 0, status = ks->status;
+    for (int it = 0; it < s.steps; ++it) {
+        struct Row {
+            T a[5], x[5];
+            int mk;
+        };
+        const double pAp = block_sum(
+            n, s.nch, sp, part,
+            [&](int i) {
+                Row v;
+                v.mk = s.mask[i];
+                const int off[5] = {-s.nx, -1, 0, 1, s.nx};
+#pragma unroll
+                for (int k = 0; k < 5; ++k) {
+                    v.a[k] = s.C[(size_t)k * n + i];
+                    v.x[k] = s.p[((v.mk >> k) & 1) ? i + off[k] : i];
+                }
+                return v;
+            },
+            [&](int i, const Row &v) {  // band_ax_at's sum
+                T ax = 0;
+#pragma unroll
+                for (int k = 0; k < 5; ++k) {
+                    const T u = ax + v.a[k] * v.x[k];
+                    ax = ((v.mk >> k) & 1) ? u : ax;
+                }
+                const T y = s.sg * ax;
+                s.Ap[i] = y;
+                return (double)v.x[2] * (double)y;
+            });
+        gprev = gamma;
+        if (pAp <= s.epsT * pn2 && fabs(pAp) <= s.epsT * pn2) {
+            done = 1;
+            status = FVH_KRYLOV_ZERO_CURV;
+            break;
+        }
+        alpha = gamma / pAp;
+        struct Alpha {
+            T x, p, r, ap;
+            int slot;
+        };
+        for (int c = 0; c < s.nch; ++c)
+            block_rows(
+                n, c, [&](int i) { return Alpha{s.x[i], s.p[i], s.r[i], s.Ap[i], s.map[i]}; },
+                [&](int i, const Alpha &v) {
+                    if (i >= n) return;
+                    s.x[i] = (double)v.x + alpha * (double)v.p;
+                    const T ri = (double)v.r + (-alpha) * (double)v.ap;
+                    s.r[i] = ri;
+                    s.bdst[(size_t)v.slot * s.stride] = ri;
+                });
+        for (int q = t; q < half; q += kCgThreads) {  // array 0 / array nw: what no wave writes
+            const int c = q / HS, j = q - c * HS;
+            fl[q] = (j == 0 || c == 0) ? T(0) : hand_sentinel<T>();
+            bl[q] = (j == 0 || c == nw) ? T(0) : hand_sentinel<T>();
+        }
+        __syncthreads();
+        if (w < nw) fwd_wave<T>(s.a, g, w, fl + w * HS, fl + (w + 1) * HS, s.recs, s.bq, s.yq);
+        __syncthreads();
+        if (w < nw) bwd_wave<T, kIlu>(s.a, g, w, bl + (w + 1) * HS, bl + w * HS, s.kb, s.yq, s.zp);
+        __syncthreads();
+        struct Pair {
+            T a, b;
+        };
+        const double gn = block_sum(
+            n, s.nch, sp, part, [&](int i) { return Pair{s.zp[s.qmap[i]], s.r[i]}; },
+            [&](int i, const Pair &v) {
+                const T zi = s.sigma * (double)v.a;
+                s.z[i] = zi;
+                return (double)v.b * (double)zi;
+            });
+        rnorm = sqrt(gn);
+        const bool solved = (rnorm <= eps) || (rnorm + 1.0 <= 1.0);
+        ++iter;
+        if (!solved) {
+            beta = gn / gprev;
+            pn2 = gn + beta * beta * pn2;
+            gamma = gn;
+        }
+        if (solved || iter >= s.itmax) {
+            done = 1;
+            status = solved ? FVH_KRYLOV_SOLVED : FVH_KRYLOV_ITMAX;
+            break;
+        }
+        for (int c = 0; c < s.nch; ++c)
+            block_rows(
+                n, c, [&](int i) { return Pair{s.z[i], s.p[i]}; },
+                [&](int i, const Pair &v) {
+                    if (i < n) s.p[i] = (double)v.a + beta * (double)v.b;
+                });
+        __syncthreads();
+    }
+    if (t == 0) {
+        ks->gamma = gamma;
+        ks->pnorm2 = pn2;
+        ks->gprev = gprev;
+        ks->alpha = alpha;
+        ks->beta = beta;
+        ks->rnorm = rnorm;
+        ks->iter = iter;
+        ks->status = status;
+        ks->done = done;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1424,6 +1630,59 @@ int skew_rhs_target(fvh_eqn *e, int fp32, SkewRhs *t) {
     }
     return FVH_OK;
 }
+
+// Grids whose CG iterations run in one work-group: the sweeps are one CU's
+// work anyway (at most three waves), so the launches around them and the gaps
+// between (25 us of kernels, 38 us elapsed an iteration on 40 x 40) become
+// barriers, until the vector work outgrows one CU or the walk of the sweeps
+// (nx + ny steps) leaves the launches no share.  us per iteration with the
+// solve's set-up, launches / one work-group:
+//             20x20      40x40      63x64      130x31     20x180     400x10
+//   FP64    39.2/19.3  43.2/24.0  52.0/40.3  48.3/39.6  62.9/59.1  73.2/66.5
+//   FP32    40.9/25.3  45.1/28.5  51.1/40.8  49.3/40.6  58.5/50.5  66.1/59.0
+// and past the limits: 1000x4 124/135 (FP32 102/101), 96x64 54/52,
+// 30x170 64/71, 127x60 53/58, 90x90 57/64, 40x190 66/96.
+constexpr int kCgSmallRows = 4096, kCgSmallWalk = 512;
+bool skew_cg_fits(const fvh_mesh *m, int fp32) {
+    if (m->cases || !skew_active(m) || m->sched.band_nx <= 0 || m->n > kCgSmallRows) return false;
+    const SkewGrid &g = m->skew->h_grids[0];
+    if (g.nx + g.ny > kCgSmallWalk) return false;
+    const SkewLayout &L = *m->skew;
+    const size_t lds = 2 * (size_t)(L.h_grids[0].nw + 1) * L.HS * (fp32 ? sizeof(float) : sizeof(double));
+    static_assert(kCgSmallRows <= kCgMaxChunks * kChunk, "block_sum");
+    return L.h_grids[0].nw <= kSkewMaxW && lds + (kCgThreads + 64) * sizeof(double) <= (size_t)max_lds_bytes();
+}
+
+template <typename T>
+int skew_cg_small(fvh_eqn *eq, const T *band, T *x, T *r, T *z, T *p, T *Ap, double sigma, double epsT, int steps,
+                  int itmax, KScal *ks) {
+    fvh_eqn *e = eq->pshare ? eq->pshare : eq;
+    const fvh_mesh *m = eq->m;
+    const SkewLayout &L = *m->skew;
+    SkewRhs rt{};
+    FVH_TRY(skew_rhs_target(e, sizeof(T) == 4, &rt));
+    SkewSweep<T> *w;
+    if constexpr (sizeof(T) == 8) w = &e->sk.s64;
+    else w = &e->sk.s32;
+    CgSmall<T> s{skew_args<Rec4T<T>>(e, 1), (int)m->n, nchunks(m->n), m->sched.band_nx, steps, itmax, rt.stride,
+                 m->sched.bmask.p, band, (T)sigma, sigma, epsT, x, r, z, p, Ap, static_cast<T *>(rt.dst), rt.map,
+                 L.qoff.p, sizeof(T) == 8 ? static_cast<const void *>(e->sk.F.p) : w->kf.p, w->bq.p, w->yq.p, w->zp.p,
+                 w->kb.p, ks};
+    const size_t lds = 2 * (size_t)(L.h_grids[0].nw + 1) * L.HS * sizeof(T);
+    if (sizeof(T) == 8 && e->sk.ilu) {
+        FVH_TRY(allow_lds(k_cg_small<T, true>, lds + (kCgThreads + 64) * sizeof(double)));
+        hipLaunchKernelGGL((k_cg_small<T, true>), dim3(1), dim3(kCgThreads), lds, stream(), s);
+    } else {
+        FVH_TRY(allow_lds(k_cg_small<T, false>, lds + (kCgThreads + 64) * sizeof(double)));
+        hipLaunchKernelGGL((k_cg_small<T, false>), dim3(1), dim3(kCgThreads), lds, stream(), s);
+    }
+    HIP_TRY(hipGetLastError());
+    return FVH_OK;
+}
+template int skew_cg_small<double>(fvh_eqn *, const double *, double *, double *, double *, double *, double *, double,
+                                   double, int, int, KScal *);
+template int skew_cg_small<float>(fvh_eqn *, const float *, float *, float *, float *, float *, float *, double, double,
+                                  int, int, KScal *);
 
 int skew_dinv_natural(fvh_eqn *e, double *out) {
     const int n = (int)e->m->n;

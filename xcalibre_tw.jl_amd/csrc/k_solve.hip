@@ -802,6 +802,8 @@ static int launch_cg_beta_spmv(fvh_eqn *e, const double *rz, KScal *ks, int itma
     return FVH_OK;
 }
 
+constexpr int kCgLaunch = 256;  // iterations of a one-work-group launch (a few ms)
+
 // An element's inputs to CG's alpha update (and its slot in the sweeps'
 // records when r goes there).
 template <typename T>
@@ -882,6 +884,15 @@ static int cg(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st, 
     const char *fuse_env = std::getenv("FVH_CG_FUSED");
     const bool fuse = !(fuse_env && fuse_env[0] == '0');
     T *pc = p, *pa = p2;
+    const T *band = sizeof(T) == 8 ? (const T *)w.bval.p : (const T *)w.bval32.p;
+    if (fuse && qmap && w.band_live && band && skew_cg_fits(e->m, sizeof(T) == 4)) {
+        while (!w.h_ks->done && enq < itmax) {
+            const int nb = std::min(kCgLaunch, itmax - enq);
+            FVH_TRY(skew_cg_small<T>(e, band, xk, r, z, p, Ap, sigma, epsT, nb, itmax, ks));
+            enq += nb;
+            FVH_TRY(read_ks(e));
+        }
+    }
     while (!w.h_ks->done && enq < itmax) {
         int nb = std::min(next_batch(enq), itmax - enq);
         for (int it = 0; it < nb; ++it) {
