@@ -508,126 +508,6 @@ static void fill_stats(fvh_eqn *e, fvh_stats *st) {
 }
 
 // ---------------------------------------------------------------------------
-// BiCGSTAB (Krylov.jl bicgstab!, left preconditioning, c = b)
-// ---------------------------------------------------------------------------
-template <typename T>
-static int bicgstab(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st) {
-    fvh_eqn *e = S.e;
-    const int n = S.n;
-    KrylovWork &w = e->kw;
-    T *xk = S.v[0], *dx = S.v[1], *r = S.v[2], *p = S.v[3], *v = S.v[4], *s = S.v[5], *q = S.v[6], *t = S.v[7];
-    const T *b = S.b;
-    double *part = w.part.p;
-    KScal *ks = w.ks.p;
-    const double atol = cfg.atol, rtol = cfg.rtol;
-    const int itmax = cfg.itmax;
-    FVH_TRY(single(ks, false, [=] __device__(KScal * k) {
-        k->done = 0;
-        k->iter = 0;
-        k->status = FVH_KRYLOV_ITMAX;
-        k->alpha = 1.0;
-        k->omega = 1.0;
-        k->rho = 1.0;
-    }));
-    if (S.warm) {
-        FVH_TRY(map(n, nullptr, [=] __device__(int i) {
-            dx[i] = xu[i];
-            xk[i] = 0;
-            s[i] = 0;
-            v[i] = 0;
-        }));
-        FVH_TRY(sys_spmv(S, dx, q, nullptr));
-        FVH_TRY(map(n, nullptr, [=] __device__(int i) { q[i] = b[i] - q[i]; }));
-    } else {
-        FVH_TRY(map(n, nullptr, [=] __device__(int i) {
-            xk[i] = 0;
-            s[i] = 0;
-            v[i] = 0;
-            q[i] = b[i];
-        }));
-    }
-    FVH_TRY(sys_precond(S, r, q, nullptr));
-    FVH_TRY(mapred<2>(n, nullptr, part, [=] __device__(int i, double(&a)[2]) {
-        p[i] = r[i];
-        a[0] = a[0] + D(r[i]) * D(r[i]);
-        a[1] = a[1] + D(b[i]) * D(r[i]);
-    }));
-    FVH_TRY(finalize<2>(n, part, ks, false, [=] __device__(KScal * k, double(&rr)[2]) {
-        double rn = sqrt(rr[0]);
-        k->rnorm = rn;
-        k->rnorm0 = rn;
-        k->eps = atol + rtol * rn;
-        k->beta = rr[1];  // next_rho
-        if (rn == 0.0) { k->done = 1; k->status = FVH_KRYLOV_ZERO_RES; return; }
-        if (rr[1] == 0.0) { k->done = 1; k->status = FVH_KRYLOV_BREAKDOWN; return; }
-        if (rn <= k->eps) { k->done = 1; k->status = FVH_KRYLOV_SOLVED; return; }
-        if (itmax <= 0) { k->done = 1; k->status = FVH_KRYLOV_ITMAX; }
-    }));
-    int enq = 0;
-    first_batch(e);
-    while (!w.h_ks->done && enq < itmax) {
-        int nb = std::min(next_batch(enq), itmax - enq);
-        for (int it = 0; it < nb; ++it) {
-            FVH_TRY(sys_spmv(S, p, q, ks));
-            FVH_TRY(sys_precond(S, v, q, ks));
-            FVH_TRY(mapred<1>(n, ks, part, [=] __device__(int i, double(&a)[1]) { a[0] = a[0] + D(b[i]) * D(v[i]); }));
-            FVH_TRY(finalize<1>(n, part, ks, true, [=] __device__(KScal * k, double(&bv)[1]) {
-                k->iter += 1;
-                k->rho = k->beta;
-                k->alpha = k->rho / bv[0];
-            }));
-            FVH_TRY(map(n, ks, [=] __device__(int i) {
-                double al = ks->alpha;
-                s[i] = D(r[i]) + (-al) * D(v[i]);
-                xk[i] = D(xk[i]) + al * D(p[i]);
-            }));
-            FVH_TRY(sys_spmv(S, s, q, ks));
-            FVH_TRY(sys_precond(S, t, q, ks));
-            FVH_TRY(mapred<2>(n, ks, part, [=] __device__(int i, double(&a)[2]) {
-                a[0] = a[0] + D(t[i]) * D(s[i]);
-                a[1] = a[1] + D(t[i]) * D(t[i]);
-            }));
-            FVH_TRY(finalize<2>(n, part, ks, true, [=] __device__(KScal * k, double(&tt)[2]) { k->omega = tt[0] / tt[1]; }));
-            FVH_TRY(mapred<2>(n, ks, part, [=] __device__(int i, double(&a)[2]) {
-                double om = ks->omega;
-                xk[i] = D(xk[i]) + om * D(s[i]);
-                const T ri = D(s[i]) + (-om) * D(t[i]);
-                r[i] = ri;
-                a[0] = a[0] + D(b[i]) * D(ri);
-                a[1] = a[1] + D(ri) * D(ri);
-            }));
-            FVH_TRY(finalize<2>(n, part, ks, true, [=] __device__(KScal * k, double(&rr)[2]) {
-                double next_rho = rr[0];
-                double beta = (next_rho / k->rho) * (k->alpha / k->omega);
-                k->beta = next_rho;
-                k->ts = beta;
-                double rn = sqrt(rr[1]);
-                k->rnorm = rn;
-                bool solved = (rn <= k->eps) || (rn + 1.0 <= 1.0);
-                bool tired = k->iter >= itmax;
-                bool brk = (k->alpha == 0.0) || isnan(k->alpha);
-                if (solved || tired || brk) {
-                    k->done = 1;
-                    k->status = solved ? FVH_KRYLOV_SOLVED : (brk ? FVH_KRYLOV_BREAKDOWN : FVH_KRYLOV_ITMAX);
-                }
-            }));
-            FVH_TRY(map(n, ks, [=] __device__(int i) {
-                double om = ks->omega, be = ks->ts;
-                double pi = D(p[i]) + (-om) * D(v[i]);
-                p[i] = D(r[i]) + be * pi;
-            }));
-        }
-        enq += nb;
-        FVH_TRY(read_ks(e));
-    }
-    if (S.warm) FVH_TRY(map(n, nullptr, [=] __device__(int i) { xu[i] = xk[i] + dx[i]; }));
-    else FVH_TRY(map(n, nullptr, [=] __device__(int i) { xu[i] = xk[i]; }));
-    if (enq == 0) FVH_TRY(read_ks(e));
-    fill_stats(e, st);
-    return FVH_OK;
-}
-
-// ---------------------------------------------------------------------------
 // CG's two scalar updates fused into the vector updates that use them.  Every
 // block reduces the partial sums itself (the canonical order of k_final, so
 // the same bits), computes the scalar and maps its elements with it; block 0
@@ -782,23 +662,269 @@ struct CsrRows {
     }
 };
 
-// The fused beta update and SpMV with the operator the system's own SpMV
+// `launch(ax)` with the row product of the operator the system's own SpMV
 // uses (banded or CSR values, FP64 or the FP32 copy).
-template <typename T>
-static int launch_cg_beta_spmv(fvh_eqn *e, const double *rz, KScal *ks, int itmax, const T *z, const T *p, T *pn,
-                               T *y, double sigma, double *part) {
+template <typename T, class L>
+static int launch_rows(fvh_eqn *e, L launch) {
     const fvh_mesh *m = e->m;
-    const int n = (int)m->n, nch = nchunks(m->n);
-    const T sg = (T)sigma;
     const T *band = sizeof(T) == 8 ? (const T *)e->kw.bval.p : (const T *)e->kw.bval32.p;
     const T *csr = sizeof(T) == 8 ? (const T *)e->nz.p : (const T *)e->kw.valf.p;
-    if (e->kw.band_live && band)
-        hipLaunchKernelGGL((k_cg_beta_spmv<T, BandRows<T>>), dim3(nch), dim3(kWide), 0, stream(), n, rz, nch, ks,
-                           itmax, z, p, pn, y, sg, part, BandRows<T>{n, m->sched.band_nx, m->sched.bmask.p, band});
-    else
-        hipLaunchKernelGGL((k_cg_beta_spmv<T, CsrRows<T>>), dim3(nch), dim3(kWide), 0, stream(), n, rz, nch, ks,
-                           itmax, z, p, pn, y, sg, part, CsrRows<T>{m->d.rowptr, m->d.col, csr});
+    if (e->kw.band_live && band) launch(BandRows<T>{(int)m->n, m->sched.band_nx, m->sched.bmask.p, band});
+    else launch(CsrRows<T>{m->d.rowptr, m->d.col, csr});
     HIP_TRY(hipGetLastError());
+    return FVH_OK;
+}
+
+// ---------------------------------------------------------------------------
+// BiCGSTAB (Krylov.jl bicgstab!, left preconditioning, c = b)
+//
+// Nine launches an iteration where each of its scalars once had a launch of
+// its own and each product a gather and a scatter (20): a block forms the
+// scalar it needs from the partial sums itself (as CG's do), the vector
+// updates p' and s run inside the products that read them (a neighbour's value
+// is formed again by the owner's expression), x takes both its updates in one
+// pass.  us per iteration with the solve's set-up, one launch each / fused,
+// DILU: FP64 40x40 90/65, 64x63 100/74, 130x90 126/100, 250x125 156/129,
+// 1000x1000 642/614; FP32 40x40 132/96, 130x90 152/114, 1000x1000 452/425.
+// ---------------------------------------------------------------------------
+// Where a product goes: natural rows, or the sweeps' right-hand side with the
+// reset of their hand-over arrays.
+template <typename T>
+struct RhsOut {
+    T *dst;
+    const int *map;  // null: natural rows
+    int stride;
+    T *hand;
+    int nhand, HS;
+    unsigned long long sent;
+    __device__ void put(int n, int i, T y) const {
+        if (map) {
+            dst[(size_t)map[i] * stride] = y;
+            for (int q = i; q < nhand; q += n) hand[q] = q % HS == 0 ? T(0) : bits_as<T>(sent);
+        } else {
+            dst[i] = y;
+        }
+    }
+};
+template <typename T>
+__device__ inline T bi_p(T r, T p, T v, double om, double be) {
+    const double pi = D(p) + (-om) * D(v);
+    return D(r) + be * pi;
+}
+// The end of an iteration from the partial sums of b.r and r.r: beta, the
+// residual norm and whether the solve stops.  Every block computes them from
+// scalars that this launch does not write; block 0 stores them.
+__device__ inline bool bi_end(const double *part, int nch, KScal *ks, int itmax, double &beta) {
+    double rr[2];
+    final_reduce<2>(part, nch, rr);
+    const double next_rho = rr[0], rn = sqrt(rr[1]), alpha = ks->alpha;
+    beta = (next_rho / ks->rho) * (alpha / ks->omega);
+    const bool solved = (rn <= ks->eps) || (rn + 1.0 <= 1.0);
+    const bool tired = ks->iter >= itmax;
+    const bool brk = (alpha == 0.0) || isnan(alpha);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ks->beta = next_rho;
+        ks->ts = beta;
+        ks->rnorm = rn;
+        if (solved || tired || brk) {
+            ks->done = 1;
+            ks->status = solved ? FVH_KRYLOV_SOLVED : (brk ? FVH_KRYLOV_BREAKDOWN : FVH_KRYLOV_ITMAX);
+        }
+    }
+    return solved || tired || brk;
+}
+// p = r + beta (p - omega v), alone (before the host reads the scalars) ...
+template <class Op>
+__global__ void __launch_bounds__(kBlock) k_bi_beta(int n, const double *part, int nch, KScal *ks, int itmax, Op op) {
+    if (block_done(ks)) return;
+    double be;
+    if (bi_end(part, nch, ks, itmax, be)) return;
+    const double om = ks->omega;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) op(i, om, be);
+}
+// ... and with the next iteration's product A p.  p' goes to a second array:
+// the old p of rows in other blocks must stay readable.
+template <typename T, class Ax>
+__global__ void __launch_bounds__(kBlock)
+    k_bi_p(int n, const double *part, int nch, KScal *ks, int itmax, const T *__restrict__ r, const T *__restrict__ p,
+           const T *__restrict__ v, T *__restrict__ pn, RhsOut<T> out, Ax ax) {
+    if (block_done(ks)) return;
+    double be;
+    if (bi_end(part, nch, ks, itmax, be)) return;
+    const double om = ks->omega;
+    const auto pnew = [=](int j) -> T { return bi_p<T>(r[j], p[j], v[j], om, be); };
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        pn[i] = pnew(i);
+        out.put(n, i, ax(pnew, i));
+    }
+}
+// alpha from the partial sums of b.v, s = r - alpha v and the product A s
+template <typename T, class Ax>
+__global__ void __launch_bounds__(kBlock)
+    k_bi_s(int n, const double *part, int nch, KScal *ks, const T *__restrict__ r, const T *__restrict__ v,
+           T *__restrict__ s, RhsOut<T> out, Ax ax) {
+    if (block_done(ks)) return;
+    double bv[1];
+    final_reduce<1>(part, nch, bv);
+    const double rho = ks->beta, al = rho / bv[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ks->iter += 1;
+        ks->rho = rho;
+        ks->alpha = al;
+    }
+    const auto snew = [=](int j) -> T { return D(r[j]) + (-al) * D(v[j]); };
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        s[i] = snew(i);
+        out.put(n, i, ax(snew, i));
+    }
+}
+// omega from the partial sums of t.s and t.t, both updates of x, r = s - omega
+// t and the partial sums of b.r and r.r: one block of kWide threads per chunk
+template <typename T>
+__global__ void __launch_bounds__(kWide)
+    k_bi_r(int n, const double *part, double *pout, int nch, KScal *ks, const T *__restrict__ b,
+           const T *__restrict__ p, const T *__restrict__ s, const T *__restrict__ t, T *__restrict__ x,
+           T *__restrict__ r) {
+    if (block_done(ks)) return;
+    double tt[2];
+    final_reduce<2>(part, nch, tt);
+    const double om = tt[0] / tt[1], al = ks->alpha;
+    if (blockIdx.x == 0 && threadIdx.x == 0) ks->omega = om;
+    __shared__ double sp[2][kChunk];
+    const int c0 = blockIdx.x * kChunk;
+#pragma unroll
+    for (int h = 0; h < kChunk / kWide; ++h) {
+        const int j = threadIdx.x + h * kWide, i = c0 + j;
+        double br = 0.0, rr = 0.0;
+        if (i < n) {
+            const T x1 = D(x[i]) + al * D(p[i]);
+            x[i] = D(x1) + om * D(s[i]);
+            const T ri = D(s[i]) + (-om) * D(t[i]);
+            r[i] = ri;
+            br = D(b[i]) * D(ri);
+            rr = D(ri) * D(ri);
+        }
+        sp[0][j] = br;
+        sp[1][j] = rr;
+    }
+    chunk_reduce_staged<2>(sp, pout, nch);
+}
+
+template <typename T>
+static int bicgstab(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st) {
+    fvh_eqn *e = S.e;
+    const int n = S.n;
+    KrylovWork &w = e->kw;
+    T *xk = S.v[0], *dx = S.v[1], *r = S.v[2], *p = S.v[3], *v = S.v[4], *s = S.v[5], *q = S.v[6], *t = S.v[7];
+    const T *b = S.b;
+    double *part = w.part.p, *part2 = w.part.p + 2 * nchunks(n);  // read and written by k_bi_r
+    KScal *ks = w.ks.p;
+    const double atol = cfg.atol, rtol = cfg.rtol;
+    const int itmax = cfg.itmax;
+    FVH_TRY(single(ks, false, [=] __device__(KScal * k) {
+        k->done = 0;
+        k->iter = 0;
+        k->status = FVH_KRYLOV_ITMAX;
+        k->alpha = 1.0;
+        k->omega = 1.0;
+        k->rho = 1.0;
+    }));
+    if (S.warm) {
+        FVH_TRY(map(n, nullptr, [=] __device__(int i) {
+            dx[i] = xu[i];
+            xk[i] = 0;
+            s[i] = 0;
+            v[i] = 0;
+        }));
+        FVH_TRY(sys_spmv(S, dx, q, nullptr));
+        FVH_TRY(map(n, nullptr, [=] __device__(int i) { q[i] = b[i] - q[i]; }));
+    } else {
+        FVH_TRY(map(n, nullptr, [=] __device__(int i) {
+            xk[i] = 0;
+            s[i] = 0;
+            v[i] = 0;
+            q[i] = b[i];
+        }));
+    }
+    FVH_TRY(sys_precond(S, r, q, nullptr));
+    FVH_TRY(mapred<2>(n, nullptr, part, [=] __device__(int i, double(&a)[2]) {
+        p[i] = r[i];
+        a[0] = a[0] + D(r[i]) * D(r[i]);
+        a[1] = a[1] + D(b[i]) * D(r[i]);
+    }));
+    FVH_TRY(finalize<2>(n, part, ks, false, [=] __device__(KScal * k, double(&rr)[2]) {
+        double rn = sqrt(rr[0]);
+        k->rnorm = rn;
+        k->rnorm0 = rn;
+        k->eps = atol + rtol * rn;
+        k->beta = rr[1];  // next_rho
+        if (rn == 0.0) { k->done = 1; k->status = FVH_KRYLOV_ZERO_RES; return; }
+        if (rr[1] == 0.0) { k->done = 1; k->status = FVH_KRYLOV_BREAKDOWN; return; }
+        if (rn <= k->eps) { k->done = 1; k->status = FVH_KRYLOV_SOLVED; return; }
+        if (itmax <= 0) { k->done = 1; k->status = FVH_KRYLOV_ITMAX; }
+    }));
+    int enq = 0;
+    // with the banded sweeps the products go straight into their layout and v
+    // and t come out of it into the dot products (as in cg)
+    const int *qmap = sys_quad_map(S);
+    RhsOut<T> out{q, nullptr, 1, nullptr, 0, 1, 0};
+    if (qmap) {
+        SkewRhs rt{};
+        FVH_TRY(sys_rhs_target(S, &rt));
+        out = RhsOut<T>{static_cast<T *>(rt.dst), rt.map, rt.stride, static_cast<T *>(rt.hand), rt.nhand, rt.HS, rt.sent};
+    }
+    const int nch = nchunks(n);
+    first_batch(e);
+    while (!w.h_ks->done && enq < itmax) {
+        int nb = std::min(next_batch(enq), itmax - enq);
+        for (int it = 0; it < nb; ++it) {
+            const T *nat = nullptr;  // the product in natural rows (its gather runs in the apply)
+            if (it > 0) {
+                T *pn = t;  // t is free until the second apply
+                FVH_TRY(launch_rows<T>(e, [&](auto ax) {
+                    hipLaunchKernelGGL(k_bi_p, fused_grid(n), dim3(kBlock), 0, stream(), n, part2, nch, ks, itmax, r,
+                                       p, v, pn, out, ax);
+                }));
+                std::swap(p, t);
+            } else {
+                FVH_TRY(sys_spmv(S, p, q, ks));
+                nat = q;
+            }
+            const T *zq = nullptr;
+            if (qmap) FVH_TRY(sys_precond_quads(S, nat, ks, &zq));
+            else FVH_TRY(sys_precond(S, v, q, ks));
+            FVH_TRY(mapred<1>(n, ks, part, [=] __device__(int i, double(&a)[1]) {
+                const T vi = qmap ? zq[qmap[i]] : v[i];
+                if (qmap) v[i] = vi;
+                a[0] = a[0] + D(b[i]) * D(vi);
+            }));
+            FVH_TRY(launch_rows<T>(e, [&](auto ax) {
+                hipLaunchKernelGGL(k_bi_s, fused_grid(n), dim3(kBlock), 0, stream(), n, part, nch, ks, r, v, s, out, ax);
+            }));
+            const T *tq = nullptr;
+            T *tt = t;
+            if (qmap) FVH_TRY(sys_precond_quads(S, nullptr, ks, &tq));
+            else FVH_TRY(sys_precond(S, t, q, ks));
+            FVH_TRY(mapred<2>(n, ks, part, [=] __device__(int i, double(&a)[2]) {
+                const T ti = qmap ? tq[qmap[i]] : tt[i];
+                if (qmap) tt[i] = ti;
+                a[0] = a[0] + D(ti) * D(s[i]);
+                a[1] = a[1] + D(ti) * D(ti);
+            }));
+            hipLaunchKernelGGL((k_bi_r<T>), dim3(nch), dim3(kWide), 0, stream(), n, part, part2, nch, ks, b, p, s, t, xk, r);
+            HIP_TRY(hipGetLastError());
+        }
+        T *pp = p;
+        hipLaunchKernelGGL(k_bi_beta, fused_grid(n), dim3(kBlock), 0, stream(), n, part2, nch, ks, itmax,
+                           [=] __device__(int i, double om, double be) { pp[i] = bi_p<T>(r[i], pp[i], v[i], om, be); });
+        HIP_TRY(hipGetLastError());
+        enq += nb;
+        FVH_TRY(read_ks(e));
+    }
+    if (S.warm) FVH_TRY(map(n, nullptr, [=] __device__(int i) { xu[i] = xk[i] + dx[i]; }));
+    else FVH_TRY(map(n, nullptr, [=] __device__(int i) { xu[i] = xk[i]; }));
+    if (enq == 0) FVH_TRY(read_ks(e));
+    fill_stats(e, st);
     return FVH_OK;
 }
 
@@ -897,7 +1023,10 @@ static int cg(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st, 
         int nb = std::min(next_batch(enq), itmax - enq);
         for (int it = 0; it < nb; ++it) {
             if (it > 0 && fuse) {
-                FVH_TRY(launch_cg_beta_spmv<T>(e, part, ks, itmax, z, pc, pa, Ap, sigma, ppap));
+                FVH_TRY(launch_rows<T>(e, [&](auto ax) {
+                    hipLaunchKernelGGL((k_cg_beta_spmv<T, decltype(ax)>), dim3(nchunks(n)), dim3(kWide), 0, stream(), n,
+                                       part, nchunks(n), ks, itmax, z, pc, pa, Ap, (T)sigma, ppap, ax);
+                }));
                 std::swap(pc, pa);
             } else {
                 if (it > 0) {
