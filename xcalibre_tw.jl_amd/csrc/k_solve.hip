@@ -490,6 +490,16 @@ static int sys_precond_quads(const Sys<double> &S, const double *x, const KScal 
 static int sys_precond_quads(const Sys<float> &S, const float *x, const KScal *ks, const float **zq) {
     return skew_apply_quads32(S.e->pshare ? S.e->pshare : S.e, x, ks, zq);
 }
+// Whether M^{-1} is elementwise, and its factors (null: the identity)
+template <typename T>
+static bool sys_diag_precond(const Sys<T> &S, const T **scale) {
+    const fvh_eqn *P = S.e->pshare ? S.e->pshare : S.e;
+    if (P->pkind == FVH_PRECOND_JACOBI || P->pkind == FVH_PRECOND_NORMDIAG) {
+        *scale = sizeof(T) == 8 ? (const T *)P->pstore.p : (const T *)P->p32a.p;
+        return true;
+    }
+    return P->pkind == FVH_PRECOND_NONE;
+}
 template <typename T>
 static int sys_rhs_target(const Sys<T> &S, SkewRhs *t) {
     return skew_rhs_target(S.e->pshare ? S.e->pshare : S.e, sizeof(T) == 4, t);
@@ -525,6 +535,25 @@ __device__ inline bool block_done(const KScal *ks) {
 }
 inline dim3 fused_grid(int64_t n) { return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((n + kBlock - 1) / kBlock, 1024))); }
 
+// alpha from the partial sums of p.Ap, or true: zero curvature, the solve stops
+__device__ inline bool cg_alpha_scalars(const double *part, int nch, KScal *ks, double epsT, double &al) {
+    double pa[1];
+    final_reduce<1>(part, nch, pa);
+    const double pAp = pa[0], gamma = ks->gamma, pn2 = ks->pnorm2;
+    const bool zc = pAp <= epsT * pn2 && fabs(pAp) <= epsT * pn2;
+    al = gamma / pAp;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ks->gprev = gamma;
+        if (zc) {
+            ks->done = 1;
+            ks->status = FVH_KRYLOV_ZERO_CURV;
+        } else {
+            ks->alpha = al;
+        }
+    }
+    return zc;
+}
+
 // alpha = gamma / pAp (or stop on zero curvature), then x += alpha p,
 // r -= alpha Ap: `load(i)` reads an element's inputs, `op(i, v, alpha)`
 // writes its results.  Each thread has at most kAlphaPer elements (the grid
@@ -544,24 +573,56 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
     for (int k = 0; k < kAlphaPer; ++k)
         if (i0 + k * stride < n) v[k] = load(i0 + k * stride);
-    double pa[1];
-    final_reduce<1>(part, nch, pa);
-    const double pAp = pa[0], gamma = ks->gamma, pn2 = ks->pnorm2;
-    const bool zc = pAp <= epsT * pn2 && fabs(pAp) <= epsT * pn2;
-    const double al = gamma / pAp;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ks->gprev = gamma;
-        if (zc) {
-            ks->done = 1;
-            ks->status = FVH_KRYLOV_ZERO_CURV;
-        } else {
-            ks->alpha = al;
-        }
-    }
-    if (zc) return;
+    double al;
+    if (cg_alpha_scalars(part, nch, ks, epsT, al)) return;
 #pragma unroll
     for (int k = 0; k < kAlphaPer; ++k)
         if (i0 + k * stride < n) op(i0 + k * stride, v[k], al);
+}
+
+// The alpha update with an elementwise preconditioner (scale: its factors,
+// null for none) and r.z in the same pass: z = sigma (scale r) and the partial
+// sums of r.z over the canonical chunks, one block of kBlock threads each, a
+// thread's rows all in flight before the reduction of p.Ap.  Bound by memory:
+8 words a row, 6.1 TB/s
+// on 1500 x 1000 (15.8 us; the alpha update, the apply and the r.z pass it
+// replaces moved 12 words in 28.5 us and three launches).  us per iteration,
+// three passes / one, Jacobi: FP64 40x40 20.3/13.6, 250x125 23.5/16.2,
+// 1000x1000 39.9/30.9, 1500x1000 56.1/43.4; FP32 1000x1000 38.8/28.1.
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    k_cg_alpha_z(int n, const double *part, int nch, KScal *ks, double epsT, double sigma, const T *__restrict__ scale,
+                 const T *__restrict__ p, const T *__restrict__ Ap, T *__restrict__ x, T *__restrict__ r,
+                 T *__restrict__ z, double *prz) {
+    if (block_done(ks)) return;
+    T vx[kPer], vp[kPer], vr[kPer], va[kPer], vs[kPer];
+    const int i0 = blockIdx.x * kChunk + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = min(i0 + k * kBlock, n - 1);
+        vx[k] = x[i];
+        vp[k] = p[i];
+        vr[k] = r[i];
+        va[k] = Ap[i];
+        vs[k] = scale ? scale[i] : T(1);
+    }
+    double al;
+    if (cg_alpha_scalars(part, nch, ks, epsT, al)) return;
+    double acc[1] = {0.0};
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = i0 + k * kBlock;
+        if (i < n) {
+            x[i] = (double)vx[k] + al * (double)vp[k];
+            const T ri = (double)vr[k] + (-al) * (double)va[k];
+            r[i] = ri;
+            const T y = scale ? vs[k] * ri : ri;
+            const T zi = sigma * (double)y;
+            z[i] = zi;
+            acc[0] = acc[0] + (double)ri * (double)zi;
+        }
+    }
+    chunk_reduce<1>(acc, prz, nch);
 }
 
 // beta = gamma_new / gamma (or stop: solved, itmax), then p = z + beta p
@@ -1003,6 +1064,9 @@ static int cg(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st, 
     const int *bmap = rt.map;
     const int bstride = rt.stride, nhand = rt.nhand, HS = rt.HS;
     const unsigned long long sent = rt.sent;
+    // an elementwise preconditioner is applied where r is updated
+    const T *scale = nullptr;
+    const bool diagM = sys_diag_precond(S, &scale);
     first_batch(e);
     // Each iteration's beta update runs fused with the next iteration's SpMV
     // (k_cg_beta_spmv, p alternating between two arrays); the last one of a
@@ -1038,6 +1102,12 @@ static int cg(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st, 
             }
             const T *pk = pc;
             const auto ld = [=] __device__(int i) { return AlphaIn<T>{xk[i], pk[i], r[i], Ap[i], qmap ? bmap[i] : 0}; };
+            if (diagM) {
+                hipLaunchKernelGGL(k_cg_alpha_z<T>, dim3(nchunks(n)), dim3(kBlock), 0, stream(), n, ppap, nchunks(n),
+                                   ks, epsT, sigma, scale, pk, Ap, xk, r, z, part);
+                HIP_TRY(hipGetLastError());
+                continue;
+            }
             if (qmap)
                 hipLaunchKernelGGL(k_cg_alpha, alpha_grid(n), dim3(kBlock), 0, stream(), (int)n, ppap, nchunks(n), ks,
                                    epsT, ld, [=] __device__(int i, const AlphaIn<T> &v, double al) {
