@@ -584,7 +584,7 @@ __global__ void __launch_bounds__(kBlock)
 // null for none) and r.z in the same pass: z = sigma (scale r) and the partial
 // sums of r.z over the canonical chunks, one block of kBlock threads each, a
 // thread's rows all in flight before the reduction of p.Ap.  Bound by memory:
-8 words a row, 6.1 TB/s
+// 8 words a row, 6.1 TB/s
 // on 1500 x 1000 (15.8 us; the alpha update, the apply and the r.z pass it
 // replaces moved 12 words in 28.5 us and three launches).  us per iteration,
 // three passes / one, Jacobi: FP64 40x40 20.3/13.6, 250x125 23.5/16.2,
