@@ -510,6 +510,11 @@ __device__ inline T bits_as(unsigned long long u) {
     else return __builtin_bit_cast(T, (unsigned)u);
 }
 
+template <typename T>
+struct Pair {
+    T a, b;
+};
+
 static void fill_stats(fvh_eqn *e, fvh_stats *st) {
     st->niter = e->kw.h_ks->iter;
     st->status = e->kw.h_ks->status;
@@ -954,11 +959,12 @@ static int bicgstab(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats
             const T *zq = nullptr;
             if (qmap) FVH_TRY(sys_precond_quads(S, nat, ks, &zq));
             else FVH_TRY(sys_precond(S, v, q, ks));
-            FVH_TRY(mapred<1>(n, ks, part, [=] __device__(int i, double(&a)[1]) {
-                const T vi = qmap ? zq[qmap[i]] : v[i];
-                if (qmap) v[i] = vi;
-                a[0] = a[0] + D(b[i]) * D(vi);
-            }));
+            FVH_TRY(mapred_wide<1>(
+                n, ks, part, [=] __device__(int i) { return Pair<T>{qmap ? zq[qmap[i]] : v[i], b[i]}; },
+                [=] __device__(int i, const Pair<T> &y, double(&a)[1]) {
+                    if (qmap) v[i] = y.a;
+                    a[0] = D(y.b) * D(y.a);
+                }));
             FVH_TRY(launch_rows<T>(e, [&](auto ax) {
                 hipLaunchKernelGGL(k_bi_s, fused_grid(n), dim3(kBlock), 0, stream(), n, part, nch, ks, r, v, s, out, ax);
             }));
@@ -966,12 +972,13 @@ static int bicgstab(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats
             T *tt = t;
             if (qmap) FVH_TRY(sys_precond_quads(S, nullptr, ks, &tq));
             else FVH_TRY(sys_precond(S, t, q, ks));
-            FVH_TRY(mapred<2>(n, ks, part, [=] __device__(int i, double(&a)[2]) {
-                const T ti = qmap ? tq[qmap[i]] : tt[i];
-                if (qmap) tt[i] = ti;
-                a[0] = a[0] + D(ti) * D(s[i]);
-                a[1] = a[1] + D(ti) * D(ti);
-            }));
+            FVH_TRY(mapred_wide<2>(
+                n, ks, part, [=] __device__(int i) { return Pair<T>{qmap ? tq[qmap[i]] : tt[i], s[i]}; },
+                [=] __device__(int i, const Pair<T> &y, double(&a)[2]) {
+                    if (qmap) tt[i] = y.a;
+                    a[0] = D(y.a) * D(y.b);
+                    a[1] = D(y.a) * D(y.a);
+                }));
             hipLaunchKernelGGL((k_bi_r<T>), dim3(nch), dim3(kWide), 0, stream(), n, part, part2, nch, ks, b, p, s, t, xk, r);
             HIP_TRY(hipGetLastError());
         }
@@ -1067,6 +1074,11 @@ static int cg(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st, 
     // an elementwise preconditioner is applied where r is updated
     const T *scale = nullptr;
     const bool diagM = sys_diag_precond(S, &scale);
+    const auto rz = [=] __device__(int i, const Pair<T> &v, double(&a)[1]) {
+        const T zi = sigma * D(v.a);
+        z[i] = zi;
+        a[0] = D(v.b) * D(zi);
+    };
     first_batch(e);
     // Each iteration's beta update runs fused with the next iteration's SpMV
     // (k_cg_beta_spmv, p alternating between two arrays); the last one of a
@@ -1127,18 +1139,10 @@ static int cg(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st, 
             if (qmap) {  // r already in the sweep layout, z read straight from the sweeps' quads
                 const T *zq = nullptr;
                 FVH_TRY(sys_precond_quads(S, nullptr, ks, &zq));
-                FVH_TRY(mapred<1>(n, ks, part, [=] __device__(int i, double(&a)[1]) {
-                    const T zi = sigma * D(zq[qmap[i]]);
-                    z[i] = zi;
-                    a[0] = a[0] + D(r[i]) * D(zi);
-                }));
+                FVH_TRY(mapred_wide<1>(n, ks, part, [=] __device__(int i) { return Pair<T>{zq[qmap[i]], r[i]}; }, rz));
             } else {
                 FVH_TRY(sys_precond(S, z, r, ks));
-                FVH_TRY(mapred<1>(n, ks, part, [=] __device__(int i, double(&a)[1]) {
-                    const T zi = sigma * D(z[i]);
-                    z[i] = zi;
-                    a[0] = a[0] + D(r[i]) * D(zi);
-                }));
+                FVH_TRY(mapred_wide<1>(n, ks, part, [=] __device__(int i) { return Pair<T>{z[i], r[i]}; }, rz));
             }
         }
         hipLaunchKernelGGL(k_cg_beta, fused_grid(n), dim3(kBlock), 0, stream(), (int)n, part, nchunks(n), ks, itmax,
@@ -1152,6 +1156,46 @@ static int cg(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st, 
     if (enq == 0) FVH_TRY(read_ks(e));
     fill_stats(e, st);
     return FVH_OK;
+}
+
+// One step of modified Gram-Schmidt: R = V_i.q from its partial sums (formed by
+// every block, stored by block 0), q -= R V_i, and the partial sums of the
+// next product V_n.q (null: q.q), into other words than it reads.  One launch
+// where the sum had a launch of its own: 4.7 us on 400 x 100
+// (a pass of about 5 and a one-block sum of about 5 before).
+template <typename T>
+__global__ void __launch_bounds__(kWide)
+    k_mgs(int n, const double *part, double *pout, int nch, const KScal *ks, double *R, const T *__restrict__ Vi,
+          const T *__restrict__ Vn, T *__restrict__ q) {
+    if (ks->done) return;
+    __shared__ double sp[1][kChunk];
+    constexpr int kRows = kChunk / kWide;
+    T vq[kRows], vi[kRows], vn[kRows];
+    const int i0 = blockIdx.x * kChunk + threadIdx.x;
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+        const int j = i0 + h * kWide;
+        if (j < n) {
+            vq[h] = q[j];
+            vi[h] = Vi[j];
+            vn[h] = Vn ? Vn[j] : T(0);
+        }
+    }
+    double d[1];
+    final_reduce<1>(part, nch, d);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *R = d[0];
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+        const int j = i0 + h * kWide;
+        double term = 0.0;
+        if (j < n) {
+            const T qj = D(vq[h]) + (-d[0]) * D(vi[h]);
+            q[j] = qj;
+            term = (Vn ? D(vn[h]) : D(qj)) * D(qj);
+        }
+        sp[0][threadIdx.x + h * kWide] = term;
+    }
+    chunk_reduce_staged<1>(sp, pout, nch);
 }
 
 // ---------------------------------------------------------------------------
@@ -1198,6 +1242,7 @@ static int gmres(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *s
     double *part = w.part.p;
     KScal *ks = w.ks.p;
     const double atol = cfg.atol, rtol = cfg.rtol;
+    double *pin = part, *pout = part + nchunks(n);
     const double btol = std::pow(std::numeric_limits<double>::epsilon(), 0.75);
     FVH_TRY(single(ks, false, [=] __device__(KScal * k) {
         k->done = 0;
@@ -1242,19 +1287,15 @@ static int gmres(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *s
             FVH_TRY(sys_spmv(S, Vk1, wv, ks));
             FVH_TRY(sys_precond(S, q, wv, ks));
             // modified Gram-Schmidt: R[nr+i] = V_i . q ; q -= R[nr+i] V_i
-            FVH_TRY(mapred<1>(n, ks, part, [=] __device__(int j, double(&a)[1]) { a[0] = a[0] + D(V[j]) * D(q[j]); }));
+            FVH_TRY(mapred_wide<1>(n, ks, pin, [=] __device__(int j) { return Pair<T>{V[j], q[j]}; },
+                                   [=] __device__(int, const Pair<T> &v, double(&a)[1]) { a[0] = D(v.a) * D(v.b); }));
             for (int i = 0; i < k; ++i) {
-                double *Ri = R + nr + i;
-                FVH_TRY(finalize<1>(n, part, ks, true, [=] __device__(KScal *, double(&d)[1]) { *Ri = d[0]; }));
-                const T *Vi = V + (size_t)i * ld;
-                const T *Vn = (i + 1 < k) ? V + (size_t)(i + 1) * ld : nullptr;
-                FVH_TRY(mapred<1>(n, ks, part, [=] __device__(int j, double(&a)[1]) {
-                    const T qj = D(q[j]) + (-(*Ri)) * D(Vi[j]);
-                    q[j] = qj;
-                    a[0] = a[0] + (Vn ? D(Vn[j]) : D(qj)) * D(qj);
-                }));
+                hipLaunchKernelGGL((k_mgs<T>), dim3(nchunks(n)), dim3(kWide), 0, stream(), n, pin, pout, nchunks(n), ks,
+                                   R + nr + i, V + (size_t)i * ld, i + 1 < k ? V + (size_t)(i + 1) * ld : nullptr, q);
+                HIP_TRY(hipGetLastError());
+                std::swap(pin, pout);
             }
-            FVH_TRY(finalize<1>(n, part, ks, true, [=] __device__(KScal * kk, double(&h)[1]) {
+            FVH_TRY(finalize<1>(n, pin, ks, true, [=] __device__(KScal * kk, double(&h)[1]) {
                 double Hbis = sqrt(h[0]);
                 for (int i = 0; i < k - 1; ++i) {
                     double Rtmp = cc[i] * R[nr + i] + ss[i] * R[nr + i + 1];
