@@ -59,8 +59,6 @@ struct SkewRhs {
     unsigned long long sent;
 };
 int skew_rhs_target(fvh_eqn *e, int fp32, SkewRhs *t);
-// the reset of the hand-over arrays alone (the gather's other half)
-int skew_hand_reset(fvh_eqn *e, int fp32);
 int skew_dinv_natural(fvh_eqn *e, double *out);
 // CG iterations of a small grid in one launch: whether the mesh's do, and up
 // to `steps` of them (band: A by band position)

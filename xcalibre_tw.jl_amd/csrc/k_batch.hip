@@ -70,6 +70,11 @@ __global__ void k_single_cases(int K, KScal *ks, bool skip, Fn fn) {
     fn(ks + k);
 }
 
+template <typename T>
+__device__ inline double D(T x) {
+    return (double)x;
+}
+
 struct Cases {
     const fvh_mesh *m;
     CaseView cv;
@@ -138,6 +143,174 @@ __global__ void __launch_bounds__(kWide) k_spmv_dot_cases(CaseView cv, const int
     chunk_reduce_staged<1>(p, part, cv.nblk);
 }
 
+// ---------------------------------------------------------------------------
+// CG's launches per case: one kWide block per (case, chunk), each forming its
+// case's scalar from the case's partial sums itself; a case's first block
+// stores it.  What a block reads from ks is not written in the same launch
+// (as CG's single-case kernels, k_solve.hip).  Five launches an iteration
+// where each sum, the beta update and the sweeps' reset had one each (nine):
+// 24 cases of 32 x 32 to
+// 256 x 256 cells, us an iteration around the sweeps: 44 in nine, 26 in five.
+// ---------------------------------------------------------------------------
+// beta, the residual norm and whether the case stops, from the sums of r.z
+__device__ inline bool cg_beta_scalars(const CaseView &cv, int b, const double *part, KScal *K, int itmax,
+                                       double &beta) {
+    const int k = cv.blk_case[b];
+    double g[1];
+    final_reduce_at<1>(part, cv.nblk, cv.cb[k], cv.cb[k + 1] - cv.cb[k], g);
+    const double gn = g[0], rn = sqrt(gn);
+    const bool solved = (rn <= K->eps) || (rn + 1.0 <= 1.0);
+    beta = gn / K->gprev;
+    if (b == cv.cb[k] && threadIdx.x == 0) {
+        K->rnorm = rn;
+        if (!solved) {
+            K->pnorm2 = gn + beta * beta * K->pnorm2;
+            K->gamma = gn;
+            K->beta = beta;
+        }
+        K->iter += 1;
+        const bool tired = K->iter >= itmax;
+        if (solved || tired) {
+            K->done = 1;
+            K->status = solved ? FVH_KRYLOV_SOLVED : FVH_KRYLOV_ITMAX;
+        }
+    }
+    return solved;  // at itmax p is updated once more: nothing reads it
+}
+// pn = z + beta p
+template <typename T>
+__global__ void __launch_bounds__(kWide)
+    k_cg_beta_cases(CaseView cv, const double *part, KScal *ks, int itmax, const T *z, const T *p, T *pn) {
+    const int b = blockIdx.x, k = cv.blk_case[b];
+    if (block_done(ks + k)) return;
+    double be;
+    if (cg_beta_scalars(cv, b, part, ks + k, itmax, be)) return;
+    const int i0 = cv.blk_row0[b] + threadIdx.x, end = cv.off[k + 1];
+#pragma unroll
+    for (int h = 0; h < kChunk / kWide; ++h)
+        if (i0 + h * kWide < end) pn[i0 + h * kWide] = D(z[i0 + h * kWide]) + be * D(p[i0 + h * kWide]);
+}
+// pn = z + beta p, y = sigma A pn and the partial sums of pn.y (into other
+// words than it reads; a neighbour's pn is formed again by the same expression)
+template <typename T>
+__global__ void __launch_bounds__(kWide)
+    k_cg_beta_spmv_cases(CaseView cv, const double *part, double *pout, KScal *ks, int itmax,
+                         const int *__restrict__ rowptr, const int *__restrict__ col, const T *__restrict__ val,
+                         const T *__restrict__ z, const T *__restrict__ p, T *__restrict__ pn, T *__restrict__ y,
+                         T sigma) {
+    const int b = blockIdx.x, k = cv.blk_case[b];
+    if (block_done(ks + k)) return;
+    double be;
+    if (cg_beta_scalars(cv, b, part, ks + k, itmax, be)) return;
+    const auto pnew = [=](int j) -> T { return D(z[j]) + be * D(p[j]); };
+    __shared__ double sp[1][kChunk];
+    const int c0 = cv.blk_row0[b], end = cv.off[k + 1];
+#pragma unroll
+    for (int h = 0; h < kChunk / kWide; ++h) {
+        const int j = threadIdx.x + h * kWide, i = c0 + j;
+        double pr = 0.0;
+        if (i < end) {
+            const T pi = pnew(i);
+            pn[i] = pi;
+            const T s = sigma * row_ax_at(rowptr, col, val, pnew, i);
+            y[i] = s;
+            pr = (double)pi * (double)s;
+        }
+        sp[0][j] = pr;
+    }
+    chunk_reduce_staged<1>(sp, pout, cv.nblk);
+}
+// alpha, x += alpha p, r -= alpha Ap, r also into the sweeps' layout (map not
+// null); the blocks past the cases' reset the hand-over arrays of every case
+template <typename T>
+__global__ void __launch_bounds__(kWide)
+    k_cg_alpha_cases(CaseView cv, const double *part, KScal *ks, double epsT, const T *__restrict__ p,
+                     const T *__restrict__ Ap, T *__restrict__ x, T *__restrict__ r, T *__restrict__ bdst,
+                     const int *__restrict__ map, int stride, T *__restrict__ hand, int nhand, int HS,
+                     unsigned long long sent) {
+    const int b = blockIdx.x;
+    if (b >= cv.nblk) {
+        const int q = (b - cv.nblk) * kWide + threadIdx.x;
+        if (q < nhand) hand[q] = q % HS == 0 ? T(0) : bits_as<T>(sent);
+        return;
+    }
+    const int k = cv.blk_case[b];
+    KScal *K = ks + k;
+    if (block_done(K)) return;
+    constexpr int kRows = kChunk / kWide;
+    T vx[kRows], vp[kRows], vr[kRows], va[kRows];
+    int slot[kRows];
+    const int i0 = cv.blk_row0[b] + threadIdx.x, end = cv.off[k + 1];
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+        const int i = i0 + h * kWide;
+        if (i < end) {
+            vx[h] = x[i];
+            vp[h] = p[i];
+            vr[h] = r[i];
+            va[h] = Ap[i];
+            slot[h] = map ? map[i] : 0;
+        }
+    }
+    double pa[1];
+    final_reduce_at<1>(part, cv.nblk, cv.cb[k], cv.cb[k + 1] - cv.cb[k], pa);
+    const double pAp = pa[0], gamma = K->gamma, pn2 = K->pnorm2;
+    const bool zc = pAp <= epsT * pn2 && fabs(pAp) <= epsT * pn2;
+    const double al = gamma / pAp;
+    if (b == cv.cb[k] && threadIdx.x == 0) {
+        K->gprev = gamma;
+        if (zc) {
+            K->done = 1;
+            K->status = FVH_KRYLOV_ZERO_CURV;
+        } else {
+            K->alpha = al;
+        }
+    }
+    if (zc) return;
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+        const int i = i0 + h * kWide;
+        if (i < end) {
+            x[i] = D(vx[h]) + al * D(vp[h]);
+            const T ri = D(vr[h]) + (-al) * D(va[h]);
+            r[i] = ri;
+            if (map) bdst[(size_t)slot[h] * stride] = ri;
+        }
+    }
+}
+// z = sigma z, read through qmap where it is not null, and the partial sums of r.z
+template <typename T>
+__global__ void __launch_bounds__(kWide)
+    k_cg_rz_cases(CaseView cv, const KScal *ks, double sigma, const int *qmap, const T *zin, T *z, const T *r,
+                  double *part) {
+    const int b = blockIdx.x, k = cv.blk_case[b];
+    if (ks[k].done) return;
+    __shared__ double sp[1][kChunk];
+    constexpr int kRows = kChunk / kWide;
+    T vz[kRows], vr[kRows];
+    const int i0 = cv.blk_row0[b] + threadIdx.x, end = cv.off[k + 1];
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+        const int i = i0 + h * kWide;
+        if (i < end) {
+            vz[h] = zin[qmap ? qmap[i] : i];
+            vr[h] = r[i];
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+        const int i = i0 + h * kWide;
+        double term = 0.0;
+        if (i < end) {
+            const T zi = sigma * D(vz[h]);
+            z[i] = zi;
+            term = D(vr[h]) * D(zi);
+        }
+        sp[0][threadIdx.x + h * kWide] = term;
+    }
+    chunk_reduce_staged<1>(sp, part, cv.nblk);
+}
+
 __global__ void __launch_bounds__(kWide) k_residual_part_cases(CaseView cv, const int *__restrict__ rowptr,
                                                                const int *__restrict__ col,
                                                                const double *__restrict__ val,
@@ -195,11 +368,6 @@ struct CSys {
 };
 
 template <typename T>
-__device__ inline double D(T x) {
-    return (double)x;
-}
-
-template <typename T>
 static int c_spmv(const CSys<T> &S, const T *x, T *y, const KScal *ks) {
     const fvh_mesh *m = S.e->m;
     hipLaunchKernelGGL((k_spmv_cases<T>), grid1d(S.C.n), dim3(256), 0, stream(), S.C.n, S.C.cv.cell_case, m->d.rowptr,
@@ -223,9 +391,8 @@ static int c_precond(const CSys<float> &S, float *y, const float *x, const KScal
 }
 // With the pipelined banded DILU, CG writes r into the sweep layout in its
 // alpha update and reads z from the sweeps' result quads (no gather or
-// scatter pass; the hand-over arrays are reset by a launch of their own,
-// since the per-case maps skip finished cases): the map of rows into the
-// quads, or null
+// scatter pass; that launch also resets the hand-over arrays of every case):
+// the map of rows into the quads, or null
 template <typename T>
 static const int *c_quad_map(const CSys<T> &S) {
     const fvh_eqn *P = S.e->pshare ? S.e->pshare : S.e;
@@ -235,12 +402,10 @@ static const int *c_quad_map(const CSys<T> &S) {
 }
 static int c_precond_quads(const CSys<double> &S, const KScal *ks, const double **zq) {
     fvh_eqn *P = S.e->pshare ? S.e->pshare : S.e;
-    FVH_TRY(skew_hand_reset(P, 0));
     return skew_apply_quads(P, nullptr, ks, zq);
 }
 static int c_precond_quads(const CSys<float> &S, const KScal *ks, const float **zq) {
     fvh_eqn *P = S.e->pshare ? S.e->pshare : S.e;
-    FVH_TRY(skew_hand_reset(P, 1));
     return skew_apply_quads32(P, nullptr, ks, zq);
 }
 
@@ -448,9 +613,10 @@ static int cg_c(const CSys<T> &S, const fvh_solver_cfg &cfg, T *xu, double sigma
     fvh_eqn *e = S.e;
     const Cases &C = S.C;
     KrylovWork &w = e->kw;
-    T *xk = S.v[0], *dx = S.v[1], *r = S.v[2], *z = S.v[3], *p = S.v[4], *Ap = S.v[5];
+    T *xk = S.v[0], *dx = S.v[1], *r = S.v[2], *z = S.v[3], *p = S.v[4], *Ap = S.v[5], *p2 = S.v[6];
     const T *b = S.b;
-    double *part = w.part.p;
+    // partial sums of r.z, and of p.Ap after them
+    double *part = w.part.p, *ppap = w.part.p + C.cv.nblk;
     KScal *ks = w.ks.p;
     const double atol = cfg.atol, rtol = cfg.rtol;
     const int itmax = cfg.itmax;
@@ -496,69 +662,32 @@ static int cg_c(const CSys<T> &S, const fvh_solver_cfg &cfg, T *xu, double sigma
     const int *qmap = c_quad_map(S);
     SkewRhs rt{};
     if (qmap) FVH_TRY(skew_rhs_target(e->pshare ? e->pshare : e, sizeof(T) == 4, &rt));
-    T *bdst = static_cast<T *>(rt.dst);
-    const int *bmap = rt.map;
-    const int bstride = rt.stride;
+    // p alternates between two arrays; a body starts and ends with it in the first
     auto body = [&](int nb) -> int {
+        T *pc = p, *pa = p2;
         for (int it = 0; it < nb; ++it) {
-            FVH_TRY(c_spmv_dot(S, p, Ap, sigma, ks, p, part));
-            FVH_TRY(C.finalize<1>(part, ks, true, [=] __device__(KScal * k, double(&pa)[1]) {
-                double pAp = pa[0];
-                if (pAp <= epsT * k->pnorm2 && fabs(pAp) <= epsT * k->pnorm2) {
-                    k->done = 1;
-                    k->status = FVH_KRYLOV_ZERO_CURV;
-                    return;
-                }
-                k->alpha = k->gamma / pAp;
-            }));
-            if (qmap) {  // r also into the sweep layout; z from the result quads
-                FVH_TRY(C.map(ks, [=] __device__(int i, const KScal *K) {
-                    double al = K->alpha;
-                    xk[i] = D(xk[i]) + al * D(p[i]);
-                    const T ri = D(r[i]) + (-al) * D(Ap[i]);
-                    r[i] = ri;
-                    bdst[(size_t)bmap[i] * bstride] = ri;
-                }));
-                const T *zq = nullptr;
-                FVH_TRY(c_precond_quads(S, ks, &zq));
-                FVH_TRY(C.mapred<1>(ks, part, [=] __device__(int i, double(&a)[1], const KScal *) {
-                    const T zi = sigma * D(zq[qmap[i]]);
-                    z[i] = zi;
-                    a[0] = a[0] + D(r[i]) * D(zi);
-                }));
+            if (it > 0) {
+                hipLaunchKernelGGL((k_cg_beta_spmv_cases<T>), dim3(C.cv.nblk), dim3(kWide), 0, stream(), C.cv, part, ppap,
+                                   ks, itmax, e->m->d.rowptr, e->m->d.col, S.val, z, pc, pa, Ap, (T)sigma);
+                HIP_TRY(hipGetLastError());
+                std::swap(pc, pa);
             } else {
-                FVH_TRY(C.map(ks, [=] __device__(int i, const KScal *K) {
-                    double al = K->alpha;
-                    xk[i] = D(xk[i]) + al * D(p[i]);
-                    r[i] = D(r[i]) + (-al) * D(Ap[i]);
-                }));
-                FVH_TRY(c_precond(S, z, r, ks));
-                FVH_TRY(C.mapred<1>(ks, part, [=] __device__(int i, double(&a)[1], const KScal *) {
-                    const T zi = sigma * D(z[i]);
-                    z[i] = zi;
-                    a[0] = a[0] + D(r[i]) * D(zi);
-                }));
+                FVH_TRY(c_spmv_dot(S, pc, Ap, sigma, ks, pc, ppap));
             }
-            FVH_TRY(C.finalize<1>(part, ks, true, [=] __device__(KScal * k, double(&g)[1]) {
-                double gn = g[0];
-                double rn = sqrt(gn);
-                k->rnorm = rn;
-                bool solved = (rn <= k->eps) || (rn + 1.0 <= 1.0);
-                if (!solved) {
-                    double beta = gn / k->gamma;
-                    k->pnorm2 = gn + beta * beta * k->pnorm2;
-                    k->gamma = gn;
-                    k->beta = beta;
-                }
-                k->iter += 1;
-                bool tired = k->iter >= itmax;
-                if (solved || tired) {
-                    k->done = 1;
-                    k->status = solved ? FVH_KRYLOV_SOLVED : FVH_KRYLOV_ITMAX;
-                }
-            }));
-            FVH_TRY(C.map(ks, [=] __device__(int i, const KScal *K) { p[i] = D(z[i]) + K->beta * D(p[i]); }));
+            hipLaunchKernelGGL((k_cg_alpha_cases<T>), dim3(C.cv.nblk + (qmap ? (rt.nhand + kWide - 1) / kWide : 0)),
+                               dim3(kWide), 0, stream(), C.cv, ppap, ks, epsT, pc, Ap, xk, r, static_cast<T *>(rt.dst),
+                               rt.map, rt.stride, static_cast<T *>(rt.hand), rt.nhand, rt.HS, rt.sent);
+            HIP_TRY(hipGetLastError());
+            const T *zin = z;
+            if (qmap) FVH_TRY(c_precond_quads(S, ks, &zin));
+            else FVH_TRY(c_precond(S, z, r, ks));
+            hipLaunchKernelGGL((k_cg_rz_cases<T>), dim3(C.cv.nblk), dim3(kWide), 0, stream(), C.cv, ks, sigma, qmap, zin,
+                               z, r, part);
+            HIP_TRY(hipGetLastError());
         }
+        hipLaunchKernelGGL((k_cg_beta_cases<T>), dim3(C.cv.nblk), dim3(kWide), 0, stream(), C.cv, part, ks, itmax, z, pc,
+                           p);
+        HIP_TRY(hipGetLastError());
         return FVH_OK;
     };
     FVH_TRY(iterate_cases(e, graph_key("cg", cfg, sizeof(T) == 4, sigma), itmax, body));

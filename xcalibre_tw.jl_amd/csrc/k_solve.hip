@@ -504,11 +504,6 @@ template <typename T>
 static int sys_rhs_target(const Sys<T> &S, SkewRhs *t) {
     return skew_rhs_target(S.e->pshare ? S.e->pshare : S.e, sizeof(T) == 4, t);
 }
-template <typename T>
-__device__ inline T bits_as(unsigned long long u) {
-    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, u);
-    else return __builtin_bit_cast(T, (unsigned)u);
-}
 
 template <typename T>
 struct Pair {
@@ -532,12 +527,6 @@ static void fill_stats(fvh_eqn *e, fvh_stats *st) {
 // from those, so every block takes the same path.  The `done` flag is read
 // once per block, before the block-wide reduction.
 // ---------------------------------------------------------------------------
-__device__ inline bool block_done(const KScal *ks) {
-    __shared__ int d;
-    if (threadIdx.x == 0) d = ks->done;
-    __syncthreads();
-    return d != 0;
-}
 inline dim3 fused_grid(int64_t n) { return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((n + kBlock - 1) / kBlock, 1024))); }
 
 // alpha from the partial sums of p.Ap, or true: zero curvature, the solve stops

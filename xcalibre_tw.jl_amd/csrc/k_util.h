@@ -82,6 +82,19 @@ __device__ inline void final_reduce(const double *__restrict__ part, int nch, do
     final_reduce_at<NV>(part, nch, 0, nch, r);
 }
 
+// `done` as the whole block sees it, where a block of the same launch may set it
+__device__ inline bool block_done(const KScal *ks) {
+    __shared__ int d;
+    if (threadIdx.x == 0) d = ks->done;
+    __syncthreads();
+    return d != 0;
+}
+template <typename T>
+__device__ inline T bits_as(unsigned long long u) {
+    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, u);
+    else return __builtin_bit_cast(T, (unsigned)u);
+}
+
 // Elementwise work + partial sums over the canonical chunk mapping.
 template <int NV, class Op>
 __global__ void __launch_bounds__(kBlock) k_mapred(int n, const KScal *ks, double *part, int nch, Op op) {
