@@ -64,7 +64,7 @@ int skew_dinv_natural(fvh_eqn *e, double *out);
 // to `steps` of them (band: A by band position)
 bool skew_cg_fits(const fvh_mesh *m, int fp32);
 template <typename T>
-int skew_cg_small(fvh_eqn *e, const T *band, T *x, T *r, T *z, T *p, T *Ap, double sigma, double epsT, int steps,
+int skew_cg_small(fvh_eqn *e, const T *band, T *x, T *r, T *p, double sigma, double epsT, int steps,
                   int itmax, KScal *ks);
 // reports (once) a sweep whose hand-over wait ran out
 int skew_check(fvh_eqn *e);

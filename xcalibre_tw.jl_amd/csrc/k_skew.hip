@@ -1015,49 +1015,47 @@ constexpr int kCgThreads = 256;     // one wave per SIMD: two would leave the sw
 constexpr int kCgMaxChunks = 2;
 static_assert(kCgThreads == kBlock, "thread = lane of the canonical reduction");
 
-// Rows of a chunk in groups of kPer per thread: all a group's loads (load(i))
-// are in flight before the first of its results (use(i, v)) is formed.  Rows
-// past n re-read the last one and are dropped.
-template <class Load, class Use>
-__device__ inline void block_rows(int n, int c, Load load, Use use) {
-    decltype(load(0)) v[kPer];
-    const int i0 = c * kChunk + threadIdx.x;
+constexpr int kCgRows = kCgMaxChunks * kPer;  // rows of a thread: t + 256 k
+
+// f(k, i) for the thread's rows, in order, unrolled (what f keeps per row
+// stays in registers); nch bounds the chunks that exist.
+template <class F>
+__device__ inline void block_rows(int n, int nch, F f) {
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) v[k] = load(min(i0 + k * kCgThreads, n - 1));
+    for (int c = 0; c < kCgMaxChunks; ++c)
+        if (c < nch) {
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) use(i0 + k * kCgThreads, v[k]);
+            for (int k = 0; k < kPer; ++k) {
+                const int i = threadIdx.x + (c * kPer + k) * kCgThreads;
+                if (i < n) f(c * kPer + k, i);
+            }
+        }
 }
 
-// Canonical sum over rows of term(i, load(i)), from every thread of the block:
-// chunk by chunk as chunk_reduce forms the partials (lane t adds rows t +
-// 256 k in order), then as final_reduce adds at most kCgMaxChunks of them
+// Canonical sum of the thread's per-chunk sums acc (lane t's rows t + 256 k in
+// order), from every thread of the block: the chunks' trees as chunk_reduce
+// forms the partials, then as final_reduce adds at most kCgMaxChunks of them
 // (lane t of its tree holds partial t, and the lanes beyond are zeros).
-template <class Load, class Term>
-__device__ inline double block_sum(int n, int nch, double *sp, double *part, Load load, Term term) {
-    const int t = threadIdx.x;
-    for (int c = 0; c < nch; ++c) {
-        double acc = 0.0;
-        block_rows(n, c, load, [&](int i, const decltype(load(0)) &v) {
-            if (i < n) acc = acc + term(i, v);
-        });
-        sp[t] = acc;
-        __syncthreads();
-        if (t < 128) sp[t] = sp[t] + sp[t + 128];
-        __syncthreads();
-        if (t < 64) {
-            double v = sp[t] + sp[t + 64];
-            v = v + __shfl_down(v, 32);
-            v = v + __shfl_down(v, 16);
-            v = v + __shfl_down(v, 8);
-            v = v + __shfl_down(v, 4);
-            v = v + __shfl_down(v, 2);
-            v = v + __shfl_down(v, 1);
-            if (t == 0) part[c] = v;
-        }
-        __syncthreads();
+__device__ inline double block_sum(const double (&acc)[kCgMaxChunks], double (&sp)[kCgMaxChunks][kCgThreads],
+                                   double *part) {
+    const int t = threadIdx.x, c = t >> 6;
+#pragma unroll
+    for (int q = 0; q < kCgMaxChunks; ++q) sp[q][t] = acc[q];
+    __syncthreads();
+    if (c < kCgMaxChunks) {  // a wave per chunk
+        const int l = t & 63;
+        double v = (sp[c][l] + sp[c][l + 128]) + (sp[c][l + 64] + sp[c][l + 192]);
+        v = v + __shfl_down(v, 32);
+        v = v + __shfl_down(v, 16);
+        v = v + __shfl_down(v, 8);
+        v = v + __shfl_down(v, 4);
+        v = v + __shfl_down(v, 2);
+        v = v + __shfl_down(v, 1);
+        if (l == 0) part[c] = v;
     }
+    __syncthreads();
     static_assert(kCgMaxChunks == 2, "the tree's last level");
-    return (0.0 + part[0]) + (nch > 1 ? 0.0 + part[1] : 0.0);
+    return (0.0 + part[0]) + (0.0 + part[1]);  // a chunk that does not exist summed to +0
 }
 
 template <typename T>
@@ -1068,61 +1066,84 @@ struct CgSmall {
     const T *C;                     // A by band position
     T sg;                           // sigma as the SpMV applies it ...
     double sigma, epsT;             // ... and as the recurrence does
-    T *x, *r, *z, *p, *Ap, *bdst;   // bdst[map[i] * stride]: the forward sweep's right-hand side
+    T *x, *r, *p, *bdst;            // bdst[map[i] * stride]: the forward sweep's right-hand side
     const int *map, *qmap;
     const void *recs;
     T *bq, *yq, *zp;
     const T *kb;
     KScal *ks;
 };
+// LDS of k_cg_small in T: the hand-over arrays of both sweeps, x, r and p
+constexpr size_t kCgStatic = (kCgMaxChunks * kCgThreads + 64) * sizeof(double);  // its reductions, rounded up
+static size_t cg_small_lds(int nw, int HS, int64_t n) { return 2 * (size_t)(nw + 1) * HS + 3 * (size_t)n; }
 
 // Up to `steps` CG iterations, expression for expression and sum for sum those
 // of cg() (k_solve.hip) with its kernels (k_cg_alpha, k_cg_beta,
-// k_spmv_dot_band, k_mapred), so the bits are the same.  p holds the next
-// iteration's direction at the end of each one.
+// k_spmv_dot_band, k_mapred_wide), so the bits are the same.  Bound by the
+// latency of each phase between two barriers: x, r and p stay in LDS, A p and z
+// in registers, and what a phase reads from memory it asks for before the one
+// that precedes it ends.  p holds the next iteration's direction at the end of
+// each iteration.
 template <typename T, bool kIlu>
 __global__ void __launch_bounds__(kCgThreads) k_cg_small(CgSmall<T> s) {
     extern __shared__ unsigned char skew_lds[];
-    __shared__ double sp[kCgThreads], part[kCgMaxChunks];
+    __shared__ double sp[kCgMaxChunks][kCgThreads], part[kCgMaxChunks];
     KScal *ks = s.ks;
     if (ks->done) return;
     const SkewGrid g = s.a.grids[0];
-    const int HS = s.a.HS, nw = g.nw, t = threadIdx.x, n = s.n, half = (nw + 1) * HS;
+    const int HS = s.a.HS, nw = g.nw, t = threadIdx.x, n = s.n, nch = s.nch, half = (nw + 1) * HS;
     T *fl = reinterpret_cast<T *>(skew_lds), *bl = fl + half;  // hand-over arrays of the two sweeps
+    T *x = bl + half, *r = x + n, *p = r + n;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     double gamma = ks->gamma, pn2 = ks->pnorm2, gprev = ks->gprev, alpha = ks->alpha, beta = ks->beta,
            rnorm = ks->rnorm;
     const double eps = ks->eps;
     int iter = ks->iter, done = 0, status = ks->status;
+    block_rows(n, nch, [&](int, int i) {
+        x[i] = s.x[i];
+        r[i] = s.r[i];
+        p[i] = s.p[i];
+    });
+    __syncthreads();
     for (int it = 0; it < s.steps; ++it) {
-        struct Row {
-            T a[5], x[5];
-            int mk;
-        };
-        const double pAp = block_sum(
-            n, s.nch, sp, part,
-            [&](int i) {
-                Row v;
-                v.mk = s.mask[i];
-                const int off[5] = {-s.nx, -1, 0, 1, s.nx};
+        T v[kCgRows];  // A p, then z
+        int slot[kCgRows];
+        double acc[kCgMaxChunks];
 #pragma unroll
-                for (int k = 0; k < 5; ++k) {
-                    v.a[k] = s.C[(size_t)k * n + i];
-                    v.x[k] = s.p[((v.mk >> k) & 1) ? i + off[k] : i];
-                }
-                return v;
-            },
-            [&](int i, const Row &v) {  // band_ax_at's sum
-                T ax = 0;
+        for (int c = 0; c < kCgMaxChunks; ++c) {
+            acc[c] = 0.0;
+            if (c < nch) {
+                T a[kPer][5];
+                int mk[kPer];
+                const int i0 = c * kChunk + t;
 #pragma unroll
-                for (int k = 0; k < 5; ++k) {
-                    const T u = ax + v.a[k] * v.x[k];
-                    ax = ((v.mk >> k) & 1) ? u : ax;
+                for (int k = 0; k < kPer; ++k) {  // rows past n re-read the last one and are dropped
+                    const int i = min(i0 + k * kCgThreads, n - 1);
+                    mk[k] = s.mask[i];
+#pragma unroll
+                    for (int q = 0; q < 5; ++q) a[k][q] = s.C[(size_t)q * n + i];
+                    slot[c * kPer + k] = s.map[i];
                 }
-                const T y = s.sg * ax;
-                s.Ap[i] = y;
-                return (double)v.x[2] * (double)y;
-            });
+#pragma unroll
+                for (int k = 0; k < kPer; ++k) {  // band_ax_at's sum
+                    const int i = min(i0 + k * kCgThreads, n - 1);
+                    const int off[5] = {-s.nx, -1, 0, 1, s.nx};
+                    T ax = 0, pi = 0;
+#pragma unroll
+                    for (int q = 0; q < 5; ++q) {
+                        const bool in = (mk[k] >> q) & 1;
+                        const T pv = p[in ? i + off[q] : i];
+                        const T u = ax + a[k][q] * pv;
+                        ax = in ? u : ax;
+                        if (q == 2) pi = pv;
+                    }
+                    const T y = s.sg * ax;
+                    v[c * kPer + k] = y;
+                    if (i0 + k * kCgThreads < n) acc[c] = acc[c] + (double)pi * (double)y;
+                }
+            }
+        }
+        const double pAp = block_sum(acc, sp, part);
         gprev = gamma;
         if (pAp <= s.epsT * pn2 && fabs(pAp) <= s.epsT * pn2) {
             done = 1;
@@ -1130,20 +1151,12 @@ __global__ void __launch_bounds__(kCgThreads) k_cg_small(CgSmall<T> s) {
             break;
         }
         alpha = gamma / pAp;
-        struct Alpha {
-            T x, p, r, ap;
-            int slot;
-        };
-        for (int c = 0; c < s.nch; ++c)
-            block_rows(
-                n, c, [&](int i) { return Alpha{s.x[i], s.p[i], s.r[i], s.Ap[i], s.map[i]}; },
-                [&](int i, const Alpha &v) {
-                    if (i >= n) return;
-                    s.x[i] = (double)v.x + alpha * (double)v.p;
-                    const T ri = (double)v.r + (-alpha) * (double)v.ap;
-                    s.r[i] = ri;
-                    s.bdst[(size_t)v.slot * s.stride] = ri;
-                });
+        block_rows(n, nch, [&](int k, int i) {
+            const T ri = (double)r[i] + (-alpha) * (double)v[k];
+            s.bdst[(size_t)slot[k] * s.stride] = ri;
+            r[i] = ri;
+            x[i] = (double)x[i] + alpha * (double)p[i];
+        });
         for (int q = t; q < half; q += kCgThreads) {  // array 0 / array nw: what no wave writes
             const int c = q / HS, j = q - c * HS;
             fl[q] = (j == 0 || c == 0) ? T(0) : hand_sentinel<T>();
@@ -1154,16 +1167,17 @@ __global__ void __launch_bounds__(kCgThreads) k_cg_small(CgSmall<T> s) {
         __syncthreads();
         if (w < nw) bwd_wave<T, kIlu>(s.a, g, w, bl + (w + 1) * HS, bl + w * HS, s.kb, s.yq, s.zp);
         __syncthreads();
-        struct Pair {
-            T a, b;
-        };
-        const double gn = block_sum(
-            n, s.nch, sp, part, [&](int i) { return Pair{s.zp[s.qmap[i]], s.r[i]}; },
-            [&](int i, const Pair &v) {
-                const T zi = s.sigma * (double)v.a;
-                s.z[i] = zi;
-                return (double)v.b * (double)zi;
-            });
+#pragma unroll
+        for (int k = 0; k < kCgRows; ++k) slot[k] = s.qmap[min(t + k * kCgThreads, n - 1)];
+#pragma unroll
+        for (int k = 0; k < kCgRows; ++k) v[k] = s.zp[slot[k]];
+#pragma unroll
+        for (int c = 0; c < kCgMaxChunks; ++c) acc[c] = 0.0;
+        block_rows(n, nch, [&](int k, int i) {
+            v[k] = s.sigma * (double)v[k];
+            acc[k / kPer] = acc[k / kPer] + (double)r[i] * (double)v[k];
+        });
+        const double gn = block_sum(acc, sp, part);
         rnorm = sqrt(gn);
         const bool solved = (rnorm <= eps) || (rnorm + 1.0 <= 1.0);
         ++iter;
@@ -1177,14 +1191,14 @@ __global__ void __launch_bounds__(kCgThreads) k_cg_small(CgSmall<T> s) {
             status = solved ? FVH_KRYLOV_SOLVED : FVH_KRYLOV_ITMAX;
             break;
         }
-        for (int c = 0; c < s.nch; ++c)
-            block_rows(
-                n, c, [&](int i) { return Pair{s.z[i], s.p[i]}; },
-                [&](int i, const Pair &v) {
-                    if (i < n) s.p[i] = (double)v.a + beta * (double)v.b;
-                });
+        block_rows(n, nch, [&](int k, int i) { p[i] = (double)v[k] + beta * (double)p[i]; });
         __syncthreads();
     }
+    block_rows(n, nch, [&](int, int i) {  // each thread its own rows
+        s.x[i] = x[i];
+        s.r[i] = r[i];
+        s.p[i] = p[i];
+    });
     if (t == 0) {
         ks->gamma = gamma;
         ks->pnorm2 = pn2;
@@ -1622,23 +1636,24 @@ int skew_rhs_target(fvh_eqn *e, int fp32, SkewRhs *t) {
 // (nx + ny steps) leaves the launches no share.  us per iteration with the
 // solve's set-up, launches / one work-group:
 //             20x20      40x40      63x64      130x31     20x180     400x10
-//   FP64    39.2/19.3  43.2/24.0  52.0/40.3  48.3/39.6  62.9/59.1  73.2/66.5
-//   FP32    40.9/25.3  45.1/28.5  51.1/40.8  49.3/40.6  58.5/50.5  66.1/59.0
-// and past the limits: 1000x4 124/135 (FP32 102/101), 96x64 54/52,
-// 30x170 64/71, 127x60 53/58, 90x90 57/64, 40x190 66/96.
+//   FP64    39.2/16.8  43.2/20.2  52.0/31.7  48.3/30.6  62.9/51.8  73.2/53.0
+//   FP32    40.9/23.1  45.1/26.1  51.1/35.5  49.3/34.5  58.5/44.0  66.1/49.2
+// Past the limits, with the vectors in memory (the LDS no longer holds them):
+// 1000x4 124/135 (FP32 102/101), 96x64 54/52, 30x170 64/71, 127x60 53/58,
+// 90x90 57/64, 40x190 66/96.
 constexpr int kCgSmallRows = 4096, kCgSmallWalk = 512;
 bool skew_cg_fits(const fvh_mesh *m, int fp32) {
     if (m->cases || !skew_active(m) || m->sched.band_nx <= 0 || m->n > kCgSmallRows) return false;
     const SkewGrid &g = m->skew->h_grids[0];
     if (g.nx + g.ny > kCgSmallWalk) return false;
     const SkewLayout &L = *m->skew;
-    const size_t lds = 2 * (size_t)(L.h_grids[0].nw + 1) * L.HS * (fp32 ? sizeof(float) : sizeof(double));
+    const size_t lds = cg_small_lds(g.nw, L.HS, m->n) * (fp32 ? sizeof(float) : sizeof(double));
     static_assert(kCgSmallRows <= kCgMaxChunks * kChunk, "block_sum");
-    return L.h_grids[0].nw <= kSkewMaxW && lds + (kCgThreads + 64) * sizeof(double) <= (size_t)max_lds_bytes();
+    return g.nw <= kSkewMaxW && lds + kCgStatic <= (size_t)max_lds_bytes();
 }
 
 template <typename T>
-int skew_cg_small(fvh_eqn *eq, const T *band, T *x, T *r, T *z, T *p, T *Ap, double sigma, double epsT, int steps,
+int skew_cg_small(fvh_eqn *eq, const T *band, T *x, T *r, T *p, double sigma, double epsT, int steps,
                   int itmax, KScal *ks) {
     fvh_eqn *e = eq->pshare ? eq->pshare : eq;
     const fvh_mesh *m = eq->m;
@@ -1649,23 +1664,23 @@ int skew_cg_small(fvh_eqn *eq, const T *band, T *x, T *r, T *z, T *p, T *Ap, dou
     if constexpr (sizeof(T) == 8) w = &e->sk.s64;
     else w = &e->sk.s32;
     CgSmall<T> s{skew_args<Rec4T<T>>(e, 1), (int)m->n, nchunks(m->n), m->sched.band_nx, steps, itmax, rt.stride,
-                 m->sched.bmask.p, band, (T)sigma, sigma, epsT, x, r, z, p, Ap, static_cast<T *>(rt.dst), rt.map,
+                 m->sched.bmask.p, band, (T)sigma, sigma, epsT, x, r, p, static_cast<T *>(rt.dst), rt.map,
                  L.qoff.p, sizeof(T) == 8 ? static_cast<const void *>(e->sk.F.p) : w->kf.p, w->bq.p, w->yq.p, w->zp.p,
                  w->kb.p, ks};
-    const size_t lds = 2 * (size_t)(L.h_grids[0].nw + 1) * L.HS * sizeof(T);
+    const size_t lds = cg_small_lds(L.h_grids[0].nw, L.HS, m->n) * sizeof(T);
     if (sizeof(T) == 8 && e->sk.ilu) {
-        FVH_TRY(allow_lds(k_cg_small<T, true>, lds + (kCgThreads + 64) * sizeof(double)));
+        FVH_TRY(allow_lds(k_cg_small<T, true>, lds + kCgStatic));
         hipLaunchKernelGGL((k_cg_small<T, true>), dim3(1), dim3(kCgThreads), lds, stream(), s);
     } else {
-        FVH_TRY(allow_lds(k_cg_small<T, false>, lds + (kCgThreads + 64) * sizeof(double)));
+        FVH_TRY(allow_lds(k_cg_small<T, false>, lds + kCgStatic));
         hipLaunchKernelGGL((k_cg_small<T, false>), dim3(1), dim3(kCgThreads), lds, stream(), s);
     }
     HIP_TRY(hipGetLastError());
     return FVH_OK;
 }
-template int skew_cg_small<double>(fvh_eqn *, const double *, double *, double *, double *, double *, double *, double,
+template int skew_cg_small<double>(fvh_eqn *, const double *, double *, double *, double *, double,
                                    double, int, int, KScal *);
-template int skew_cg_small<float>(fvh_eqn *, const float *, float *, float *, float *, float *, float *, double, double,
+template int skew_cg_small<float>(fvh_eqn *, const float *, float *, float *, float *, double, double,
                                   int, int, KScal *);
 
 int skew_dinv_natural(fvh_eqn *e, double *out) {

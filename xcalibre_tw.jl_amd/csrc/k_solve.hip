@@ -1079,7 +1079,7 @@ static int cg(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *st, 
     if (fuse && qmap && w.band_live && band && skew_cg_fits(e->m, sizeof(T) == 4)) {
         while (!w.h_ks->done && enq < itmax) {
             const int nb = std::min(kCgLaunch, itmax - enq);
-            FVH_TRY(skew_cg_small<T>(e, band, xk, r, z, p, Ap, sigma, epsT, nb, itmax, ks));
+            FVH_TRY(skew_cg_small<T>(e, band, xk, r, p, sigma, epsT, nb, itmax, ks));
             enq += nb;
             FVH_TRY(read_ks(e));
         }
