@@ -739,8 +739,11 @@ static int launch_rows(fvh_eqn *e, L launch) {
 // updates p' and s run inside the products that read them (a neighbour's value
 // is formed again by the owner's expression), x takes both its updates in one
 // pass.  us per iteration with the solve's set-up, one launch each / fused,
-// DILU: FP64 40x40 90/65, 64x63 100/74, 130x90 126/100, 250x125 156/129,
-// 1000x1000 642/614; FP32 40x40 132/96, 130x90 152/114, 1000x1000 452/425.
+// DILU: FP64 40x40 90/63, 64x63 100/68, 130x90 126/94, 250x125 156/123,
+// 1000x1000 642/625; FP32 40x40 132/95, 130x90 152/108, 1000x1000 452/420.
+// At 1M rows in FP64 k_bi_s takes 47-55 us, most of it the scatter into the
+// 32-byte records; natural rows and a gather pass came to the same (623/618 on
+// 2000x500) and cost 8 us an iteration on small grids.
 // ---------------------------------------------------------------------------
 // Where a product goes: natural rows, or the sweeps' right-hand side with the
 // reset of their hand-over arrays.
