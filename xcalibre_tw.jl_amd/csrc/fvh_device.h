@@ -38,6 +38,19 @@ constexpr int kBlock = 256;
 constexpr int kPer = 8;
 constexpr int kChunk = kBlock * kPer;
 
+// The block's place when blocks are dealt to the 8 XCDs in turn and each XCD is
+// to take a contiguous eighth of the rows: rows that share neighbours (or the
+// sweeps' records of adjacent grid rows) then meet in one L2.  A permutation of
+// 0 .. gridDim.x - 1 whatever the dealing.  us, in launch order / so placed:
+// CG's beta + SpMV on 2000x500 17.5/14.9 and on 1500x1000 24.5/21.5, r.z read
+// through the quads on 2000x500 9.6/7.5, banded SpMV on 1500x1000 16.5/13.1,
+// Green-Gauss on 250k points 12.2/10.3.  CG's alpha update (17.0/18.9) and the
+// assembly's cell pass (100.0/100.4 on 2000x1000) keep the launch order.
+__device__ inline int xcd_block() {
+    const int x = blockIdx.x & 7, q = gridDim.x >> 3, r = gridDim.x & 7;
+    return x * q + min(x, r) + (int)(blockIdx.x >> 3);
+}
+
 inline int nchunks(int64_t n) { return (int)((n + kChunk - 1) / kChunk); }
 
 hipStream_t stream();

@@ -140,7 +140,7 @@ __global__ void __launch_bounds__(kWide) k_spmv_dot_cases(CaseView cv, const int
         }
         p[0][j] = pr;
     }
-    chunk_reduce_staged<1>(p, part, cv.nblk);
+    chunk_reduce_staged<1>(p, part, cv.nblk, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(kWide)
         }
         sp[0][j] = pr;
     }
-    chunk_reduce_staged<1>(sp, pout, cv.nblk);
+    chunk_reduce_staged<1>(sp, pout, cv.nblk, blockIdx.x);
 }
 // alpha, x += alpha p, r -= alpha Ap, r also into the sweeps' layout (map not
 // null); the blocks past the cases' reset the hand-over arrays of every case
@@ -308,7 +308,7 @@ __global__ void __launch_bounds__(kWide)
         }
         sp[0][threadIdx.x + h * kWide] = term;
     }
-    chunk_reduce_staged<1>(sp, part, cv.nblk);
+    chunk_reduce_staged<1>(sp, part, cv.nblk, blockIdx.x);
 }
 
 __global__ void __launch_bounds__(kWide) k_residual_part_cases(CaseView cv, const int *__restrict__ rowptr,
@@ -331,7 +331,7 @@ __global__ void __launch_bounds__(kWide) k_residual_part_cases(CaseView cv, cons
         p[0][j] = d2;
         p[1][j] = b2;
     }
-    chunk_reduce_staged<2>(p, part, cv.nblk);
+    chunk_reduce_staged<2>(p, part, cv.nblk, blockIdx.x);
 }
 
 __global__ void __launch_bounds__(kBlock) k_residual_final_cases(CaseView cv, const double *part, double *out,

@@ -107,7 +107,7 @@ constexpr int kFaceGroup = 4;
 
 __global__ void k_green_gauss(DevMesh m, const double *__restrict__ phif, double *__restrict__ dx,
                               double *__restrict__ dy, double *__restrict__ dz) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
+    int c = xcd_block() * blockDim.x + threadIdx.x;
     if (c >= m.n) return;
     double rx = 0.0, ry = 0.0, rz = 0.0;
     const int i1 = m.cf_ptr[c + 1];

@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(kWide) k_residual_part(int n, const int *__res
                                                          const double *__restrict__ x, const double *__restrict__ b,
                                                          double *part, int nch) {
     __shared__ double p[2][kChunk];
-    const int c0 = blockIdx.x * kChunk;
+    const int blk = xcd_block(), c0 = blk * kChunk;
 #pragma unroll
     for (int h = 0; h < kChunk / kWide; ++h) {
         const int j = threadIdx.x + h * kWide, i = c0 + j;
@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(kWide) k_residual_part(int n, const int *__res
         p[0][j] = d2;
         p[1][j] = b2;
     }
-    chunk_reduce_staged<2>(p, part, nch);
+    chunk_reduce_staged<2>(p, part, nch, blk);
 }
 
 __global__ void __launch_bounds__(kBlock) k_residual_final(const double *part, int nch, int n, double *out) {
@@ -680,7 +680,7 @@ __global__ void __launch_bounds__(kWide)
     if (solved) return;
     const auto pnew = [=](int j) -> V { return (V)((double)z[j] + beta * (double)p[j]); };
     __shared__ double sp[1][kChunk];
-    const int c0 = blockIdx.x * kChunk;
+    const int blk = xcd_block(), c0 = blk * kChunk;
 #pragma unroll
     for (int h = 0; h < kChunk / kWide; ++h) {
         const int j = threadIdx.x + h * kWide, i = c0 + j;
@@ -694,7 +694,7 @@ __global__ void __launch_bounds__(kWide)
         }
         sp[0][j] = pr;
     }
-    chunk_reduce_staged<1>(sp, part, nch);
+    chunk_reduce_staged<1>(sp, part, nch, blk);
 }
 
 template <typename V>
@@ -811,7 +811,7 @@ __global__ void __launch_bounds__(kBlock)
     if (bi_end(part, nch, ks, itmax, be)) return;
     const double om = ks->omega;
     const auto pnew = [=](int j) -> T { return bi_p<T>(r[j], p[j], v[j], om, be); };
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    for (int i = xcd_block() * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         pn[i] = pnew(i);
         out.put(n, i, ax(pnew, i));
     }
@@ -831,7 +831,7 @@ __global__ void __launch_bounds__(kBlock)
         ks->alpha = al;
     }
     const auto snew = [=](int j) -> T { return D(r[j]) + (-al) * D(v[j]); };
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    for (int i = xcd_block() * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         s[i] = snew(i);
         out.put(n, i, ax(snew, i));
     }
@@ -865,7 +865,7 @@ __global__ void __launch_bounds__(kWide)
         sp[0][j] = br;
         sp[1][j] = rr;
     }
-    chunk_reduce_staged<2>(sp, pout, nch);
+    chunk_reduce_staged<2>(sp, pout, nch, blockIdx.x);
 }
 
 template <typename T>
@@ -1187,7 +1187,7 @@ __global__ void __launch_bounds__(kWide)
         }
         sp[0][threadIdx.x + h * kWide] = term;
     }
-    chunk_reduce_staged<1>(sp, pout, nch);
+    chunk_reduce_staged<1>(sp, pout, nch, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------

@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(256) k_spmv_band(int n, int nx, const unsigned
                                                    const V *__restrict__ C, const V *__restrict__ x,
                                                    V *__restrict__ y, V sigma, const KScal *ks) {
     if (ks && ks->done) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
     if (i < n) y[i] = sigma * band_ax(n, nx, mask, C, x, i);
 }
 
@@ -91,17 +91,17 @@ __global__ void __launch_bounds__(256) k_spmv(int n, const int *__restrict__ row
                                               const V *__restrict__ val, const V *__restrict__ x, V *__restrict__ y,
                                               V sigma, const KScal *ks) {
     if (ks && ks->done) return;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
     if (i < n) y[i] = sigma * row_ax(rowptr, col, val, x, i);
 }
 
 // Canonical partial sums of one 2048-row chunk from per-row terms staged in
 // LDS (p[v][j] = term of row chunk_base + j, 0 for rows past n): lane t < 256
 // adds rows t + 256 k in ascending k, then the same tree as chunk_reduce.
-// All kWide threads of the block call it.
+// blk: the chunk's place among the partials.  All kWide threads of the block call it.
 constexpr int kWide = 1024;
 template <int NV>
-__device__ inline void chunk_reduce_staged(double (&p)[NV][kChunk], double *__restrict__ part, int nch) {
+__device__ inline void chunk_reduce_staged(double (&p)[NV][kChunk], double *__restrict__ part, int nch, int blk) {
     const int t = threadIdx.x;
     __syncthreads();
     double acc[NV];
@@ -134,7 +134,7 @@ __device__ inline void chunk_reduce_staged(double (&p)[NV][kChunk], double *__re
             a = a + __shfl_down(a, 4);
             a = a + __shfl_down(a, 2);
             a = a + __shfl_down(a, 1);
-            if (t == 0) part[v * nch + blockIdx.x] = a;
+            if (t == 0) part[v * nch + blk] = a;
         }
     }
 }
@@ -151,7 +151,8 @@ __global__ void __launch_bounds__(kWide) k_mapred_wide(int n, const KScal *ks, d
     __shared__ double sp[NV][kChunk];
     constexpr int kRows = kChunk / kWide;
     decltype(load(0)) v[kRows];
-    const int i0 = blockIdx.x * kChunk + threadIdx.x;
+    const int blk = xcd_block();
+    const int i0 = blk * kChunk + threadIdx.x;
 #pragma unroll
     for (int h = 0; h < kRows; ++h)
         if (i0 + h * kWide < n) v[h] = load(i0 + h * kWide);
@@ -164,7 +165,7 @@ __global__ void __launch_bounds__(kWide) k_mapred_wide(int n, const KScal *ks, d
 #pragma unroll
         for (int q = 0; q < NV; ++q) sp[q][threadIdx.x + h * kWide] = a[q];
     }
-    chunk_reduce_staged<NV>(sp, part, nch);
+    chunk_reduce_staged<NV>(sp, part, nch, blk);
 }
 template <int NV, class Ld, class Op>
 inline int mapred_wide(int64_t n, const KScal *ks, double *part, Ld load, Op op) {
@@ -184,7 +185,8 @@ __global__ void __launch_bounds__(kWide) k_spmv_dot(int n, const int *__restrict
                                                     const V *__restrict__ w, double *part, int nch) {
     if (ks && ks->done) return;
     __shared__ double p[1][kChunk];
-    const int c0 = blockIdx.x * kChunk;
+    const int blk = xcd_block();
+    const int c0 = blk * kChunk;
 #pragma unroll
     for (int h = 0; h < kChunk / kWide; ++h) {
         const int j = threadIdx.x + h * kWide, i = c0 + j;
@@ -196,7 +198,7 @@ __global__ void __launch_bounds__(kWide) k_spmv_dot(int n, const int *__restrict
         }
         p[0][j] = pr;
     }
-    chunk_reduce_staged<1>(p, part, nch);
+    chunk_reduce_staged<1>(p, part, nch, blk);
 }
 
 // The banded k_spmv_dot.
@@ -207,7 +209,8 @@ __global__ void __launch_bounds__(kWide) k_spmv_dot_band(int n, int nx, const un
                                                          const V *__restrict__ w, double *part, int nch) {
     if (ks && ks->done) return;
     __shared__ double p[1][kChunk];
-    const int c0 = blockIdx.x * kChunk;
+    const int blk = xcd_block();
+    const int c0 = blk * kChunk;
 #pragma unroll
     for (int h = 0; h < kChunk / kWide; ++h) {
         const int j = threadIdx.x + h * kWide, i = c0 + j;
@@ -219,7 +222,7 @@ __global__ void __launch_bounds__(kWide) k_spmv_dot_band(int n, int nx, const un
         }
         p[0][j] = pr;
     }
-    chunk_reduce_staged<1>(p, part, nch);
+    chunk_reduce_staged<1>(p, part, nch, blk);
 }
 
 // A's values by band position (see band_ax) from the CSR values.
