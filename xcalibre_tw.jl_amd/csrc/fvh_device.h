@@ -45,7 +45,8 @@ constexpr int kChunk = kBlock * kPer;
 // CG's beta + SpMV on 2000x500 17.5/14.9 and on 1500x1000 24.5/21.5, r.z read
 // through the quads on 2000x500 9.6/7.5, banded SpMV on 1500x1000 16.5/13.1,
 // Green-Gauss on 250k points 12.2/10.3.  CG's alpha update (17.0/18.9) and the
-// assembly's cell pass (100.0/100.4 on 2000x1000) keep the launch order.
+// assembly's cell pass (100.0/100.4 on 2000x1000) keep the launch order, and so
+// do the CSR products (4000x1000, past the Infinity Cache: 57.4/63.6).
 __device__ inline int xcd_block() {
     const int x = blockIdx.x & 7, q = gridDim.x >> 3, r = gridDim.x & 7;
     return x * q + min(x, r) + (int)(blockIdx.x >> 3);

@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(kWide) k_residual_part(int n, const int *__res
                                                          const double *__restrict__ x, const double *__restrict__ b,
                                                          double *part, int nch) {
     __shared__ double p[2][kChunk];
-    const int blk = xcd_block(), c0 = blk * kChunk;
+    const int blk = blockIdx.x, c0 = blk * kChunk;
 #pragma unroll
     for (int h = 0; h < kChunk / kWide; ++h) {
         const int j = threadIdx.x + h * kWide, i = c0 + j;
@@ -517,6 +517,12 @@ static void fill_stats(fvh_eqn *e, fvh_stats *st) {
     st->rnorm0 = e->kw.h_ks->rnorm0;
 }
 
+// A product's place among the rows (Ax: its row product)
+template <class Ax>
+__device__ inline int row_block() {
+    return Ax::kXcd ? xcd_block() : (int)blockIdx.x;
+}
+
 // ---------------------------------------------------------------------------
 // CG's two scalar updates fused into the vector updates that use them.  Every
 // block reduces the partial sums itself (the canonical order of k_final, so
@@ -680,7 +686,7 @@ __global__ void __launch_bounds__(kWide)
     if (solved) return;
     const auto pnew = [=](int j) -> V { return (V)((double)z[j] + beta * (double)p[j]); };
     __shared__ double sp[1][kChunk];
-    const int blk = xcd_block(), c0 = blk * kChunk;
+    const int blk = row_block<Ax>(), c0 = blk * kChunk;
 #pragma unroll
     for (int h = 0; h < kChunk / kWide; ++h) {
         const int j = threadIdx.x + h * kWide, i = c0 + j;
@@ -699,6 +705,7 @@ __global__ void __launch_bounds__(kWide)
 
 template <typename V>
 struct BandRows {
+    static constexpr bool kXcd = true;
     int n, nx;
     const unsigned char *mask;
     const V *C;
@@ -709,6 +716,7 @@ struct BandRows {
 };
 template <typename V>
 struct CsrRows {
+    static constexpr bool kXcd = false;
     const int *rowptr, *col;
     const V *val;
     template <class X>
@@ -811,7 +819,7 @@ __global__ void __launch_bounds__(kBlock)
     if (bi_end(part, nch, ks, itmax, be)) return;
     const double om = ks->omega;
     const auto pnew = [=](int j) -> T { return bi_p<T>(r[j], p[j], v[j], om, be); };
-    for (int i = xcd_block() * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    for (int i = row_block<Ax>() * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         pn[i] = pnew(i);
         out.put(n, i, ax(pnew, i));
     }
@@ -831,7 +839,7 @@ __global__ void __launch_bounds__(kBlock)
         ks->alpha = al;
     }
     const auto snew = [=](int j) -> T { return D(r[j]) + (-al) * D(v[j]); };
-    for (int i = xcd_block() * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    for (int i = row_block<Ax>() * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         s[i] = snew(i);
         out.put(n, i, ax(snew, i));
     }

@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(256) k_spmv(int n, const int *__restrict__ row
                                               const V *__restrict__ val, const V *__restrict__ x, V *__restrict__ y,
                                               V sigma, const KScal *ks) {
     if (ks && ks->done) return;
-    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) y[i] = sigma * row_ax(rowptr, col, val, x, i);
 }
 
@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(kWide) k_spmv_dot(int n, const int *__restrict
                                                     const V *__restrict__ w, double *part, int nch) {
     if (ks && ks->done) return;
     __shared__ double p[1][kChunk];
-    const int blk = xcd_block();
+    const int blk = blockIdx.x;
     const int c0 = blk * kChunk;
 #pragma unroll
     for (int h = 0; h < kChunk / kWide; ++h) {
