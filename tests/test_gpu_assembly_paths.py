@@ -8,6 +8,7 @@ import pytest
 
 import fvmhip as F
 from fvmhip import _lib as L
+from oracle import ref
 from tests.cases import same_bits
 
 pytestmark = pytest.mark.gpu
@@ -57,3 +58,44 @@ def test_reference_and_boundary_passes(nx, ny):
             assert same_bits(gA, A) and same_bits(gb, b), (nx, ny, cell)
         finally:
             LIB().fvh_eqn_destroy(eq)
+
+
+def _both(spec):
+    """A term list for the device and for the oracle: (operator, scheme, sign, flux, phi)."""
+    dev, host, keep = (L.Term * len(spec))(), (L.Term * len(spec))(), []
+    for k, (op, scheme, sign, *fields) in enumerate(spec):
+        for t in (dev[k], host[k]):
+            t.op, t.scheme, t.sign = op, scheme, sign
+        for attr, a in zip(("flux", "phi"), fields):
+            if a is not None:
+                d, h = L.DeviceArray.from_host(a), np.ascontiguousarray(a)
+                keep += [d, h]
+                setattr(dev[k], attr, d.ptr)
+                setattr(host[k], attr, h.ctypes.data)
+    return dev, host, keep
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 1), (2, 1), (16, 16), (257, 3)])
+def test_a_new_term_list_replaces_the_whole_matrix(nx, ny):
+    """discretise! zeroes A first: an equation assembled before keeps nothing of
+    it, whatever the next model's terms (none of a face among them)."""
+    mesh = F.channel(nx, ny)
+    dm = mesh.device()
+    n, nf = mesh.ncells, mesh.nfaces
+    rng = np.random.default_rng(n)
+    flux, gam, si, prev = rng.standard_normal(nf), 1.0 + rng.random(nf), rng.random(n), rng.standard_normal(n)
+    face = [(L.OP_DIVERGENCE, F.Upwind, 1, flux, None), (L.OP_LAPLACIAN, F.Linear, -1, gam, None)]
+    time, source = [(L.OP_TIME, F.Euler, 1, None, None)], [(L.OP_SI, F.Linear, -1, si, prev)]
+    steady = [(L.OP_TIME, F.Steady, 1, None, None)]
+    dprev, eq = L.DeviceArray.from_host(prev), C.c_void_p()
+    none = (L.BC * 1)()
+    L.check(LIB().fvh_eqn_create(dm.h, C.byref(eq)))
+    try:
+        for spec in (face, time, face + time, source, face[:1], steady, face[1:] + source, time + source):
+            dev, host, keep = _both(spec)
+            L.check(LIB().fvh_discretise(eq, dev, len(spec), None, 0, dprev.vp, 0.25))
+            gA, gb = _arrays(eq, dm.pattern()[1].size, n)
+            A, b = ref.assemble(mesh, host, len(spec), None, 0, prev, 0.25, none, 0, 0)
+            assert same_bits(gA, A) and same_bits(gb, b), (nx, ny, [t[0] for t in spec])
+    finally:
+        LIB().fvh_eqn_destroy(eq)

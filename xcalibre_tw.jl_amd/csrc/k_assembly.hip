@@ -73,7 +73,9 @@ __global__ void __launch_bounds__(256) k_asm_cells(DevMesh m, AsmArgs a, int cou
     double diag, b;
     if (NFT >= 0) {
         diag = 0.0;
-        if (NFT > 0) {
+        if (NFT == 0) {  // no term of a face: A's entries of an earlier model go
+            for (int i = m.cf_ptr[c]; i < m.cf_ptr[c + 1]; ++i) nz[m.cf_slot[i]] = 0.0;
+        } else if (NFT > 0) {
             // four sides at a time: their index loads, then their faces'
             // loads, issued together
             constexpr int G = 4, NT = NFT > 0 ? NFT : 1;
