@@ -108,7 +108,6 @@ struct SkewStore {
     DBuf<double> uhand;
     SkewSweep<double> s64;
     SkewSweep<float> s32;
-    bool ilu = false;  // the records are ILU(0)'s
     int *h_fault = nullptr;
     SkewStore() = default;
     SkewStore(const SkewStore &) = delete;
@@ -182,11 +181,14 @@ struct fvh_eqn {
     fvh::DBuf<double> D, Dinv, lu, pstore;
     fvh::DBuf<float> p32a, p32b;  // FP32 copies: Dinv / Jacobi scale, and A or LU values
     fvh::BandStore bd;  // DILU on banded grids (packed order)
-    fvh::SkewStore sk;  // DILU on banded grids (pipelined sweeps)
+    fvh::SkewStore sk, sk_ilu;  // DILU / ILU(0) on banded grids (pipelined sweeps)
     fvh::LevelStore lv; // DILU on unstructured meshes (level-scheduled records)
     fvh::LdlStore ldl;  // LDL: factor of the set-up matrix
     fvh::KrylovWork kw;
     fvh::DBuf<double> red;  // residual reductions
+    // the sweeps' records of the preconditioner that is set (each kind keeps its own last update)
+    fvh::SkewStore &sweeps() { return pkind == FVH_PRECOND_ILU0 ? sk_ilu : sk; }
+    const fvh::SkewStore &sweeps() const { return pkind == FVH_PRECOND_ILU0 ? sk_ilu : sk; }
 };
 
 namespace fvh {

@@ -1321,7 +1321,7 @@ static const int *cell_grid(const fvh_mesh *m) { return m->cases ? m->cases->cel
 
 static int skew_alloc(fvh_eqn *e) {
     const SkewLayout &L = *e->m->skew;
-    SkewStore &s = e->sk;
+    SkewStore &s = e->sweeps();
     if (s.F.n == L.NS) return FVH_OK;
     FVH_TRY(s.F.alloc(L.NS));
     FVH_TRY(s.Bk.alloc(L.NS));
@@ -1366,7 +1366,7 @@ static int sweep_records(fvh_eqn *e, SkewSweep<T> &w) {
     const SkewLayout &L = *e->m->skew;
     FVH_TRY(sweep_alloc(w, L));
     hipLaunchKernelGGL((k_skew_quads<T>), dim3((unsigned)((most_quads(L) + 255) / 256), (unsigned)L.h_grids.size()),
-                       dim3(256), 0, stream(), L.grids.p, e->sk.F.p, e->sk.Bk.p, w.kf.p, w.kb.p);
+                       dim3(256), 0, stream(), L.grids.p, e->sweeps().F.p, e->sweeps().Bk.p, w.kf.p, w.kb.p);
     HIP_TRY(hipGetLastError());
     return FVH_OK;
 }
@@ -1375,7 +1375,7 @@ template <typename R>
 static SkewArgs skew_args(const fvh_eqn *e, int W) {
     const SkewLayout &L = *e->m->skew;
     return SkewArgs{L.grids.p, L.blk_grid[W - 1].p, L.nblk[W - 1], L.HS, e->m->cases ? 1 : 0,
-                    (unsigned)(L.NS * sizeof(R)), e->sk.h_fault};
+                    (unsigned)(L.NS * sizeof(R)), e->sweeps().h_fault};
 }
 
 // Dynamic LDS beyond 64 KiB has to be allowed per kernel.
@@ -1390,10 +1390,11 @@ static int allow_lds(K kernel, size_t bytes) {
 template <int W, bool kIlu>
 static int launch_update_w(fvh_eqn *e) {
     const SkewLayout &L = *e->m->skew;
+    const SkewStore &s = e->sweeps();
     const size_t lds = (size_t)(W + 1) * L.HS * sizeof(double);
     FVH_TRY(allow_lds(k_skew_update<W, kIlu>, lds));
     hipLaunchKernelGGL((k_skew_update<W, kIlu>), dim3(L.nblk[W - 1]), dim3(64 * (W + 2)), lds, stream(),
-                       skew_args<Rec4>(e, W), e->sk.U.p, e->sk.F.p, e->sk.Bk.p, e->sk.uhand.p);
+                       skew_args<Rec4>(e, W), s.U.p, s.F.p, s.Bk.p, s.uhand.p);
     HIP_TRY(hipGetLastError());
     return FVH_OK;
 }
@@ -1406,11 +1407,11 @@ static int skew_factor(fvh_eqn *e, const double *val) {
     fvh_mesh *m = e->m;
     const SkewLayout &L = *m->skew;
     FVH_TRY(skew_alloc(e));
-    e->sk.ilu = kIlu;
+    const SkewStore &s = e->sweeps();
     const int n = (int)m->n, nhand = L.nblk[0] * L.HS;
     hipLaunchKernelGGL((k_skew_pack<kIlu>), grid_for(std::max(n, nhand)), dim3(256), 0, stream(), n, L.grids.p,
-                       cell_grid(m), L.slot_of.p, m->d.rowptr, m->d.diag, val, e->sk.F.p, e->sk.Bk.p, e->sk.U.p,
-                       e->sk.uhand.p, nhand, L.HS);
+                       cell_grid(m), L.slot_of.p, m->d.rowptr, m->d.diag, val, s.F.p, s.Bk.p, s.U.p, s.uhand.p,
+                       nhand, L.HS);
     HIP_TRY(hipGetLastError());
     switch (skew_waves(L)) {
         case 1: return launch_update_w<1, kIlu>(e);
@@ -1426,9 +1427,9 @@ int skew_update(fvh_eqn *e, const double *val) {
     int edge = 0;
     for (const SkewGrid &g : L.h_grids) edge = std::max(edge, g.nx + g.ny);
     hipLaunchKernelGGL(k_skew_edges, dim3((unsigned)((edge + 255) / 256), (unsigned)L.h_grids.size()), dim3(256), 0,
-                       stream(), L.grids.p, e->sk.F.p, e->sk.Bk.p);
+                       stream(), L.grids.p, e->sweeps().F.p, e->sweeps().Bk.p);
     HIP_TRY(hipGetLastError());
-    FVH_TRY(sweep_records(e, e->sk.s64));
+    FVH_TRY(sweep_records(e, e->sweeps().s64));
     if (!m->skew->W && !forced_waves()) FVH_TRY(skew_tune(e));
     return FVH_OK;
 }
@@ -1436,11 +1437,12 @@ int skew_update(fvh_eqn *e, const double *val) {
 int skew_ilu_update(fvh_eqn *e, const double *val) {
     const SkewLayout &L = *e->m->skew;
     FVH_TRY(skew_factor<true>(e, val));
-    FVH_TRY(sweep_alloc(e->sk.s64, L));
+    SkewStore &s = e->sweeps();
+    FVH_TRY(sweep_alloc(s.s64, L));
     hipLaunchKernelGGL(k_skew_ilu, dim3((unsigned)((most_quads(L) + 255) / 256), (unsigned)L.h_grids.size()), dim3(256),
-                       0, stream(), L.grids.p, e->sk.F.p, e->sk.Bk.p, e->sk.s64.kb.p);
+                       0, stream(), L.grids.p, s.F.p, s.Bk.p, s.s64.kb.p);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_skew_unit_pivots, grid_for(L.NS), dim3(256), 0, stream(), L.NS, e->sk.F.p);
+    hipLaunchKernelGGL(k_skew_unit_pivots, grid_for(L.NS), dim3(256), 0, stream(), L.NS, s.F.p);
     HIP_TRY(hipGetLastError());
     if (!e->m->skew->W && !forced_waves()) FVH_TRY(skew_tune(e));
     return FVH_OK;
@@ -1453,7 +1455,8 @@ int skew_ilu_update(fvh_eqn *e, const double *val) {
 // flag), so that the two equations' solves can run at the same time.
 int skew_copy(fvh_eqn *e, const fvh_eqn *src) {
     const SkewLayout &L = *e->m->skew;
-    if (src->m != e->m || src->sk.F.n != L.NS || src->sk.s64.kb.n != (size_t)kBwdN * L.NS)
+    if (src->m != e->m || e->pkind != FVH_PRECOND_DILU || src->pkind != FVH_PRECOND_DILU || src->sk.F.n != L.NS ||
+        src->sk.s64.kb.n != (size_t)kBwdN * L.NS)
         return set_error(FVH_ERR_ARG, "DILU records not prepared");
     FVH_TRY(skew_alloc(e));
     FVH_TRY(sweep_alloc(e->sk.s64, L));
@@ -1471,7 +1474,7 @@ static int launch_sweeps_w(fvh_eqn *e, SkewSweep<T> &w, const KScal *ks) {
     const size_t lds = (size_t)(W + 1) * L.HS * sizeof(T), lds_f = lds;
     FVH_TRY(allow_lds(k_skew_fwd<T, W>, lds_f));
     FVH_TRY(allow_lds(k_skew_bwd<T, W, kIlu>, lds));
-    const void *recs = sizeof(T) == 8 ? static_cast<const void *>(e->sk.F.p) : w.kf.p;
+    const void *recs = sizeof(T) == 8 ? static_cast<const void *>(e->sweeps().F.p) : w.kf.p;
     hipLaunchKernelGGL((k_skew_fwd<T, W>), dim3(a.nblk), dim3(64 * (W + 2)), lds_f, stream(), a, recs, w.bq.p, w.yq.p,
                        w.hand.p, ks);
     HIP_TRY(hipGetLastError());
@@ -1485,7 +1488,7 @@ static int launch_sweeps_w(fvh_eqn *e, SkewSweep<T> &w, const KScal *ks) {
 template <typename T, int W>
 static int launch_sweeps_k(fvh_eqn *e, SkewSweep<T> &w, const KScal *ks) {
     if constexpr (sizeof(T) == 8) {
-        if (e->sk.ilu) return launch_sweeps_w<T, W, true>(e, w, ks);
+        if (e->pkind == FVH_PRECOND_ILU0) return launch_sweeps_w<T, W, true>(e, w, ks);
     }
     return launch_sweeps_w<T, W, false>(e, w, ks);
 }
@@ -1505,7 +1508,7 @@ static int skew_sweeps_t(fvh_eqn *e, const T *x, const KScal *ks, SkewSweep<T> &
         const int ntiles = (int)L.tiles.n;
         hipLaunchKernelGGL((k_skew_gather<T>), dim3(ntiles + (nhand + 255) / 256), dim3(256), 0, stream(), ntiles,
                            L.tiles.p, L.grids.p, x,
-                           sizeof(T) == 8 ? reinterpret_cast<Rec4T<T> *>(e->sk.F.p) : nullptr, w.bq.p, w.hand.p,
+                           sizeof(T) == 8 ? reinterpret_cast<Rec4T<T> *>(e->sweeps().F.p) : nullptr, w.bq.p, w.hand.p,
                            nhand, L.HS, ks_all);
         HIP_TRY(hipGetLastError());
     }
@@ -1565,40 +1568,41 @@ static int skew_tune_t(fvh_eqn *e, SkewSweep<T> &w, int &W_out) {
 }
 
 static int skew_tune(fvh_eqn *e) {
-    return skew_tune_t<double>(e, e->sk.s64, e->m->skew->W);
+    return skew_tune_t<double>(e, e->sweeps().s64, e->m->skew->W);
 }
 
 int skew_apply(fvh_eqn *e, const double *x, double *y, const KScal *ks) {
-    SkewStore &s = e->sk;
-    if (!s.s64.kf.p) return set_error(FVH_ERR_ARG, "DILU records not prepared");
+    SkewStore &s = e->sweeps();
+    if (!s.s64.kf.p) return set_error(FVH_ERR_ARG, "sweep records not prepared (no update yet)");
     return skew_apply_t<double>(e, x, y, ks, s.s64);
 }
 
 bool skew_tuned32(const fvh_mesh *m) { return forced_waves() || m->skew->W32 != 0; }
 
 int skew_to32(fvh_eqn *e) {
-    SkewStore &s = e->sk;
+    SkewStore &s = e->sweeps();
+    if (!s.s64.kf.p) return set_error(FVH_ERR_ARG, "sweep records not prepared (no update yet)");
     FVH_TRY(sweep_records(e, s.s32));
     if (!e->m->skew->W32 && !forced_waves()) FVH_TRY(skew_tune_t<float>(e, s.s32, e->m->skew->W32));
     return FVH_OK;
 }
 
 int skew_apply32(fvh_eqn *e, const float *x, float *y, const KScal *ks) {
-    SkewStore &s = e->sk;
+    SkewStore &s = e->sweeps();
     if (!s.s32.kf.p) return set_error(FVH_ERR_ARG, "FP32 sweep records not prepared");
     return skew_apply_t<float>(e, x, y, ks, s.s32);
 }
 
 int skew_apply_quads(fvh_eqn *e, const double *x, const KScal *ks, const double **zq) {
-    SkewStore &s = e->sk;
-    if (!s.s64.kf.p) return set_error(FVH_ERR_ARG, "DILU records not prepared");
+    SkewStore &s = e->sweeps();
+    if (!s.s64.kf.p) return set_error(FVH_ERR_ARG, "sweep records not prepared (no update yet)");
     FVH_TRY(skew_sweeps_t<double>(e, x, ks, s.s64));
     *zq = s.s64.zp.p;
     return FVH_OK;
 }
 
 int skew_apply_quads32(fvh_eqn *e, const float *x, const KScal *ks, const float **zq) {
-    SkewStore &s = e->sk;
+    SkewStore &s = e->sweeps();
     if (!s.s32.kf.p) return set_error(FVH_ERR_ARG, "FP32 sweep records not prepared");
     FVH_TRY(skew_sweeps_t<float>(e, x, ks, s.s32));
     *zq = s.s32.zp.p;
@@ -1609,21 +1613,22 @@ const int *skew_quad_map(const fvh_mesh *m) { return m->skew ? m->skew->qoff.p :
 
 int skew_rhs_target(fvh_eqn *e, int fp32, SkewRhs *t) {
     const SkewLayout &L = *e->m->skew;
+    const SkewStore &s = e->sweeps();
     t->nhand = 2 * L.nblk[0] * L.HS;
     t->HS = L.HS;
     if (fp32) {
-        if (!e->sk.s32.bq.p) return set_error(FVH_ERR_ARG, "FP32 sweep records not prepared");
-        t->dst = e->sk.s32.bq.p;
+        if (!s.s32.bq.p) return set_error(FVH_ERR_ARG, "FP32 sweep records not prepared");
+        t->dst = s.s32.bq.p;
         t->map = L.qoff.p;
         t->stride = 1;
-        t->hand = e->sk.s32.hand.p;
+        t->hand = s.s32.hand.p;
         t->sent = HandWord<float>::kSent;
     } else {
-        if (!e->sk.F.p) return set_error(FVH_ERR_ARG, "DILU records not prepared");
-        t->dst = e->sk.F.p;  // b is word 0 of each 4-word record
+        if (!s.F.p) return set_error(FVH_ERR_ARG, "sweep records not prepared (no update yet)");
+        t->dst = s.F.p;  // b is word 0 of each 4-word record
         t->map = L.slot_of.p;
         t->stride = 4;
-        t->hand = e->sk.s64.hand.p;
+        t->hand = s.s64.hand.p;
         t->sent = HandWord<double>::kSent;
     }
     return FVH_OK;
@@ -1660,15 +1665,16 @@ int skew_cg_small(fvh_eqn *eq, const T *band, T *x, T *r, T *p, double sigma, do
     const SkewLayout &L = *m->skew;
     SkewRhs rt{};
     FVH_TRY(skew_rhs_target(e, sizeof(T) == 4, &rt));
+    SkewStore &st = e->sweeps();
     SkewSweep<T> *w;
-    if constexpr (sizeof(T) == 8) w = &e->sk.s64;
-    else w = &e->sk.s32;
+    if constexpr (sizeof(T) == 8) w = &st.s64;
+    else w = &st.s32;
     CgSmall<T> s{skew_args<Rec4T<T>>(e, 1), (int)m->n, nchunks(m->n), m->sched.band_nx, steps, itmax, rt.stride,
                  m->sched.bmask.p, band, (T)sigma, sigma, epsT, x, r, p, static_cast<T *>(rt.dst), rt.map,
-                 L.qoff.p, sizeof(T) == 8 ? static_cast<const void *>(e->sk.F.p) : w->kf.p, w->bq.p, w->yq.p, w->zp.p,
+                 L.qoff.p, sizeof(T) == 8 ? static_cast<const void *>(st.F.p) : w->kf.p, w->bq.p, w->yq.p, w->zp.p,
                  w->kb.p, ks};
     const size_t lds = cg_small_lds(L.h_grids[0].nw, L.HS, m->n) * sizeof(T);
-    if (sizeof(T) == 8 && e->sk.ilu) {
+    if (sizeof(T) == 8 && e->pkind == FVH_PRECOND_ILU0) {
         FVH_TRY(allow_lds(k_cg_small<T, true>, lds + kCgStatic));
         hipLaunchKernelGGL((k_cg_small<T, true>), dim3(1), dim3(kCgThreads), lds, stream(), s);
     } else {
@@ -1685,6 +1691,7 @@ template int skew_cg_small<float>(fvh_eqn *, const float *, float *, float *, fl
 
 int skew_dinv_natural(fvh_eqn *e, double *out) {
     const int n = (int)e->m->n;
+    if (!e->sk.F.p) return set_error(FVH_ERR_ARG, "sweep records not prepared (no update yet)");
     hipLaunchKernelGGL(k_skew_dinv_natural, grid_for(n), dim3(256), 0, stream(), n, e->m->skew->slot_of.p, e->sk.F.p,
                        out);
     HIP_TRY(hipGetLastError());
@@ -1697,11 +1704,12 @@ int skew_dinv_natural(fvh_eqn *e, double *out) {
 int skew_check(fvh_eqn *e) {
     fvh_eqn *owners[2] = {e, e->pshare};
     for (fvh_eqn *q : owners) {
-        int *f = q ? q->sk.h_fault : nullptr;
-        if (f && __atomic_load_n(f, __ATOMIC_ACQUIRE)) {
-            __atomic_store_n(f, 0, __ATOMIC_RELEASE);
-            return set_error(FVH_ERR_HIP, "band sweep: a hand-over between waves did not arrive in time");
-        }
+        if (!q) continue;
+        for (int *f : {q->sk.h_fault, q->sk_ilu.h_fault})
+            if (f && __atomic_load_n(f, __ATOMIC_ACQUIRE)) {
+                __atomic_store_n(f, 0, __ATOMIC_RELEASE);
+                return set_error(FVH_ERR_HIP, "band sweep: a hand-over between waves did not arrive in time");
+            }
     }
     return FVH_OK;
 }
@@ -1713,7 +1721,7 @@ int skew_check(fvh_eqn *e) {
 extern "C" int fvh_precond_fault(fvh_eqn *e, int32_t raise, int32_t *pending) {
     if (!e) return fvh::set_error(FVH_ERR_ARG, "null equation");
     fvh_eqn *q = e->pshare ? e->pshare : e;
-    int *f = q->sk.h_fault;
+    int *f = q->sweeps().h_fault;
     if (!f) return fvh::set_error(FVH_ERR_UNSUPPORTED, "the equation's preconditioner has no pipelined sweeps");
     if (raise) __atomic_store_n(f, 1, __ATOMIC_RELEASE);
     if (pending) *pending = __atomic_load_n(f, __ATOMIC_ACQUIRE);
