@@ -1,5 +1,6 @@
 """ILU(0) and DILU on the band sweeps keep records of their own: an update, or
-a set-up, of one leaves nothing in the other's."""
+a set-up, of one leaves nothing in the other's, and an update leaves nothing of
+the matrix before it."""
 import ctypes as C
 
 import numpy as np
@@ -56,6 +57,30 @@ def _inputs(nx, ny):
 
 
 SIZES = [(7, 1), (1, 7), (20, 12), (65, 65), (130, 70)]
+
+
+@pytest.mark.parametrize("nx,ny", SIZES)
+@pytest.mark.parametrize("kind", [L.PRECOND_DILU, L.PRECOND_ILU0])
+def test_an_update_forgets_a_singular_matrix(kind, nx, ny):
+    """No entries, a zero pivot and a NaN, each followed by a regular matrix:
+    the applies are those of a fresh equation."""
+    mesh, dm, (A, _), x, on_diag = _inputs(nx, ny)
+    n = mesh.ncells
+    with _Eq(dm, n) as fresh, _Eq(dm, n) as used:
+        for eq in (fresh, used):
+            eq.set(kind)
+        fresh.update(A)
+        want = fresh.apply(x), fresh.apply(x, True)
+        assert np.isfinite(want[0]).all() and np.isfinite(want[1]).all()
+        zero, nan = A.copy(), A.copy()
+        zero[np.nonzero(on_diag)[0][n // 2]] = 0.0
+        nan[np.nonzero(on_diag)[0][n - 1]] = np.nan
+        for bad in (np.zeros_like(A), zero, nan):
+            used.update(bad)
+            used.apply(x), used.apply(x, True)
+            used.update(A)
+            assert same_bits(used.apply(x), want[0]), (kind, nx, ny)
+            assert same_bits(used.apply(x, True), want[1]), (kind, nx, ny)
 
 
 @pytest.mark.parametrize("nx,ny", SIZES)

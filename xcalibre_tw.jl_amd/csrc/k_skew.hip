@@ -975,7 +975,9 @@ __global__ void k_skew_quads(const SkewGrid *__restrict__ grids, Rec4 *__restric
 // D_w into F (the division the factorization makes of the row's entry), 1 / D
 // into Bk.b (the FP32 quads) and (D, A_re, A_rn) into the backward quads.  F.b
 // is only read here (a row's west pivot is another thread's): the next kernel
-// sets it to the forward sweep's pivot, 1.
+// sets it to the forward sweep's pivot, 1.  Padding keeps its zero coefficients
+// and gets the pivot 1, whatever the recurrence left there: next to a zero or
+// NaN pivot that is a NaN, which would stay in slots that no packing rewrites.
 __global__ void k_skew_ilu(const SkewGrid *__restrict__ grids, Rec4 *__restrict__ F, Rec4 *__restrict__ Bk,
                            double *__restrict__ kb) {
     const SkewGrid g = grids[blockIdx.y];
@@ -987,10 +989,14 @@ __global__ void k_skew_ilu(const SkewGrid *__restrict__ grids, Rec4 *__restrict_
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         const size_t s = s0 + (size_t)w * g.S;
-        const double d = F[s].b, dw = F[s - g.S].b;
+        const int i = 4 * qi + w - kSkewQ0 - j;  // the row's cell on this diagonal
+        const bool cell = j < g.ny && i >= 0 && i < g.nx;
+        const double d = cell ? F[s].b : 1.0, dw = F[s - g.S].b;
         const Rec4 v = Bk[s];
-        F[s].c = F[s].c / d;
-        F[s].d = F[s].d / dw;
+        if (cell) {
+            F[s].c = F[s].c / d;
+            F[s].d = F[s].d / (i > 0 ? dw : 1.0);
+        }
         Bk[s].b = 1.0 / d;
         kb[kBwdN * (o + w)] = d;
         kb[kBwdN * (o + w) + 1] = v.c;
