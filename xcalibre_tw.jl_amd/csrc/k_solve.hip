@@ -1587,10 +1587,12 @@ extern "C" int fvh_precond_set(fvh_eqn *e, int32_t kind, fvh_eqn *matrix_of) {
 }
 
 extern "C" int fvh_precond_update(fvh_eqn *e) {
+    FVH_GUARD_BEGIN
     if (!e) return set_error(FVH_ERR_ARG, "null equation");
     FVH_TRY(precond_update(e));
     HIP_TRY(hipStreamSynchronize(stream()));
     return fault_check(e);
+    FVH_GUARD_END
 }
 
 extern "C" int fvh_precond_apply(fvh_eqn *e, double *y, const double *x) {

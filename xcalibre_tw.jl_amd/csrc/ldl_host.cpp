@@ -20,8 +20,8 @@
 #include <array>
 #include <atomic>
 #include <cmath>
+#include <exception>
 #include <numeric>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -287,22 +287,32 @@ void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out
     f.inv.resize(off[ng]);
     b.inv.resize(off[ng]);
     std::atomic<int> next{0};
-    const auto invert = [&] {
-        std::vector<double> X;
-        for (int g0; (g0 = next.fetch_add(64)) < ng;)
-            for (int g = g0; g < std::min(g0 + 64, ng); ++g)
-                invert_range(F, cut[g], cut[g + 1] - cut[g], X, whole[g], &f.inv[0] + off[g], &b.inv[0] + off[g]);
+    const int nt = off[ng] < (1 << 17) ? 1 : std::max(1, std::min(8, (int)std::thread::hardware_concurrency()));
+    std::vector<std::exception_ptr> failed(nt);  // an exception must not leave a thread, nor pass running ones
+    const auto invert = [&](int t) {
+        try {
+            std::vector<double> X;
+            for (int g0; (g0 = next.fetch_add(64)) < ng;)
+                for (int g = g0; g < std::min(g0 + 64, ng); ++g)
+                    invert_range(F, cut[g], cut[g + 1] - cut[g], X, whole[g], f.inv.data() + off[g],
+                                 b.inv.data() + off[g]);
+        } catch (...) {
+            failed[t] = std::current_exception();
+            next = ng;
+        }
     };
     {
-        const int nt = off[ng] < (1 << 17) ? 1 : std::max(1, std::min(8, (int)std::thread::hardware_concurrency()));
         std::vector<std::thread> th;
+        th.reserve(nt);
         try {
-            for (int k = 1; k < nt; ++k) th.emplace_back(invert);
-        } catch (const std::system_error &) {  // fewer threads then
+            for (int t = 1; t < nt; ++t) th.emplace_back(invert, t);
+        } catch (...) {  // fewer threads then
         }
-        invert();
+        invert(0);
         for (auto &t : th) t.join();
     }
+    for (const auto &e : failed)
+        if (e) std::rethrow_exception(e);
     // a range's parent in the tree holds the first of its outside rows; a
     // block's gates are words of the (at most two highest) ranges right below
     // it (forward) or of the parent (backward)
