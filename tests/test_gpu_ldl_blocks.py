@@ -52,3 +52,22 @@ def test_block_solves_against_substitution(nx, ny, monkeypatch):
     print(f"{nx}x{ny}: residual {res:.1e} (substitution {res0:.1e}), difference {diff:.1e}", flush=True)
     # the difference is the residuals' times the condition number (<= 8.05 / 0.05)
     assert res <= 1e-13 and diff <= 1e-11
+
+
+@pytest.mark.parametrize("nx,ny", [(13, 5), (70, 66), (310, 140)])
+@pytest.mark.parametrize("shift", [0.5, 1.3, 2.7])
+def test_indefinite_matrices(nx, ny, shift, monkeypatch):
+    """Ranges cut where their inverse grows (down to single rows): the residual
+    is the substitution's.  Two solves of like accuracy differ by a factor of
+    about e^0.6 either way; 8 is more than three of that (uncut, 310 x 140 and
+    1.3: 11 times the substitution's)."""
+    mesh = F.channel(nx, ny)
+    dm = mesh.device()
+    rp, ci = dm.pattern()
+    rows = np.repeat(np.arange(mesh.ncells), np.diff(rp))
+    vals = np.where(rows == ci, 4.0 - shift, -1.0)
+    x = np.random.default_rng(nx).standard_normal(mesh.ncells)
+    got, res = _apply(dm, vals, x, monkeypatch, True)
+    want, res0 = _apply(dm, vals, x, monkeypatch, False)
+    print(f"{nx}x{ny} {shift}: residual {res:.1e} (substitution {res0:.1e})", flush=True)
+    assert res <= 8 * res0

@@ -28,3 +28,11 @@ def test_a_failed_allocation_reaches_the_caller(checker, nx, ny):
     """One thread (small factors) and several: never the end of the process."""
     r = checker("alloc", nx, ny)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+
+
+@pytest.mark.parametrize("nx,ny", [(9, 7), (70, 66), (310, 140)])
+def test_block_solves_round_as_the_substitution_does(checker, nx, ny):
+    """Growth of a range's inverse cuts the range: no less accurate than the
+    substitution on indefinite matrices either."""
+    r = checker("solve", nx, ny)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)

@@ -202,7 +202,11 @@ int ldl_factor(int n, const int *rowptr, const int *col, const double *val, cons
 // Inverse of the unit lower triangular block of s rows from r0, packed
 // without its unit diagonal by rows (row i: columns 0 .. i-1) and by columns
 // (column k: rows k+1 .. s-1), into the sides that read it so.  X: scratch.
-static void invert_range(const LdlHost &F, int r0, int s, std::vector<double> &X, bool whole, double *f, double *b) {
+// Where an entry is above kLdlGrowth, the row it is in goes to `cuts`: between
+// two cuts every entry is within it.  (A diagonal block of the inverse is the
+// inverse of that block.)
+static void invert_range(const LdlHost &F, int r0, int s, std::vector<double> &X, bool whole, double *f, double *b,
+                         std::vector<int> &cuts) {
     if (X.size() < (size_t)s * s) X.resize((size_t)s * s);
     // X starts as the block itself (below its diagonal); row i of the inverse
     // then replaces row i: -sum_k L_ik (row k of the inverse), k ascending (L_ik
@@ -211,6 +215,7 @@ static void invert_range(const LdlHost &F, int r0, int s, std::vector<double> &X
     for (int k = 0; k < s; ++k)
         for (int p = F.Lp[r0 + k]; p < F.Lp[r0 + k + 1] && F.Li[p] < r0 + s; ++p)
             X[(size_t)(F.Li[p] - r0) * s + k] = F.Lx[p];
+    int from = 0;
     for (int i = 1; i < s; ++i) {
         double *xi = &X[(size_t)i * s];
         for (int k = 0; k < i; ++k) {
@@ -220,6 +225,12 @@ static void invert_range(const LdlHost &F, int r0, int s, std::vector<double> &X
             for (int c = 0; c < k; ++c) xi[c] -= l * xk[c];
             xi[k] = -l;
         }
+        for (int c = from; c < i; ++c)
+            if (!(std::fabs(xi[c]) <= kLdlGrowth)) {  // (a NaN too)
+                cuts.push_back(r0 + i);
+                from = i;
+                break;
+            }
     }
     double *rows = whole ? b : f, *cols = whole ? f : b;  // a whole range: lane = row, column after column
     for (int i = 1; i < s; ++i)
@@ -228,12 +239,10 @@ static void invert_range(const LdlHost &F, int r0, int s, std::vector<double> &X
         for (int i = k + 1; i < s; ++i) *cols++ = X[(size_t)i * s + k];
 }
 
-void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out) {
-    const int n = F.n;
-    std::vector<int> cut{0};
-    for (size_t g = 0; g + 1 < bounds.size(); ++g)
-        for (int a = bounds[g]; a < bounds[g + 1]; a += kLdlRange) cut.push_back(std::min(a + kLdlRange, bounds[g + 1]));
-    const int ng = (int)cut.size() - 1;
+// The blocks of the ranges between `cut`; rows that a range has to be cut at
+// as well, for the growth of its inverse, go to `more`.
+static void blocks_of(const LdlHost &F, const std::vector<int> &cut, LdlBlocks &out, std::vector<int> &more) {
+    const int n = F.n, ng = (int)cut.size() - 1;
     std::vector<int> range_of(n);
     for (int g = 0; g < ng; ++g)
         for (int i = cut[g]; i < cut[g + 1]; ++i) range_of[i] = g;
@@ -288,6 +297,7 @@ void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out
     b.inv.resize(off[ng]);
     std::atomic<int> next{0};
     const int nt = off[ng] < (1 << 17) ? 1 : std::max(1, std::min(8, (int)std::thread::hardware_concurrency()));
+    std::vector<std::vector<int>> cuts(nt);
     std::vector<std::exception_ptr> failed(nt);  // an exception must not leave a thread, nor pass running ones
     const auto invert = [&](int t) {
         try {
@@ -295,7 +305,7 @@ void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out
             for (int g0; (g0 = next.fetch_add(64)) < ng;)
                 for (int g = g0; g < std::min(g0 + 64, ng); ++g)
                     invert_range(F, cut[g], cut[g + 1] - cut[g], X, whole[g], f.inv.data() + off[g],
-                                 b.inv.data() + off[g]);
+                                 b.inv.data() + off[g], cuts[t]);
         } catch (...) {
             failed[t] = std::current_exception();
             next = ng;
@@ -313,6 +323,8 @@ void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out
     }
     for (const auto &e : failed)
         if (e) std::rethrow_exception(e);
+    for (const auto &c : cuts) more.insert(more.end(), c.begin(), c.end());
+    if (!more.empty()) return;
     // a range's parent in the tree holds the first of its outside rows; a
     // block's gates are words of the (at most two highest) ranges right below
     // it (forward) or of the parent (backward)
@@ -345,8 +357,22 @@ void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out
             for (int i = 0; i < s; i += kLdlWaves) blk.push_back({2, r0 + i, r0, s, {r0, r0 + s - 1}, off[g]});
         }
     };
+    f.blocks.clear();
+    b.blocks.clear();
     list(hf, true, f.blocks);
     list(hb, false, b.blocks);
+}
+
+void ldl_blocks(const LdlHost &F, const std::vector<int> &bounds, LdlBlocks &out) {
+    std::vector<int> cut{0}, more;
+    for (size_t g = 0; g + 1 < bounds.size(); ++g)
+        for (int a = bounds[g]; a < bounds[g + 1]; a += kLdlRange) cut.push_back(std::min(a + kLdlRange, bounds[g + 1]));
+    blocks_of(F, cut, out, more);
+    if (more.empty()) return;
+    cut.insert(cut.end(), more.begin(), more.end());
+    std::sort(cut.begin(), cut.end());
+    more.clear();
+    blocks_of(F, cut, out, more);  // the same inverses in smaller pieces: nothing more to cut
 }
 
 }  // namespace fvh
