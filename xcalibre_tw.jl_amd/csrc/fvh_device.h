@@ -104,8 +104,7 @@ struct DevMesh {
     int n, nf, nbf, nnz, ncf;
     const int *rowptr, *col, *diag, *tslot;         // CSR pattern of A
     const int *cf_ptr, *cf_face, *cf_nbr, *cf_slot;  // cell -> internal faces (faces_range order)
-    const double *cf_sign, *cf_w, *cf_omw;           // nsign, divergence weights of that side
-    int nif;                                         // internal faces (faces nbf .. nf-1)
+    const double *cf_w;                              // divergence weight of that side
     const int *cf_fs;                                // cf_face with the side's nsign: f, or ~f when it is -1
     const int *own1, *own2;                          // face owners (boundary: own1 == own2)
     const double *fw, *farea, *fdelta;               // face weight, area, delta
@@ -280,7 +279,7 @@ struct fvh_mesh {
         bf_face, bf_cell, bf_patch, cf_fs, fb_patch;
     fvh::DBuf<double> ex, ey, ez;
     bool cf_ascending = true;  // every cell's internal faces in ascending face id
-    fvh::DBuf<double> cf_sign, cf_w, cf_omw, fw, farea, fdelta, Sfx, Sfy, Sfz, nx, ny, nz, vol, ccx, ccy, ccz, fcx,
+    fvh::DBuf<double> cf_w, fw, farea, fdelta, Sfx, Sfy, Sfz, nx, ny, nz, vol, ccx, ccy, ccz, fcx,
         fcy, fcz;
     // host copies used by set-up code
     std::vector<int> h_rowptr, h_col, h_diag, h_bf_face, h_bf_cell, h_bf_patch;

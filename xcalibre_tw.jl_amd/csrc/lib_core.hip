@@ -417,7 +417,7 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
         }
     std::vector<int> cf_slot(ncf);
     std::vector<char> used(nnz, 0);
-    std::vector<double> cf_w(ncf), cf_omw(ncf);
+    std::vector<double> cf_w(ncf);
     for (int c = 0; c < n; ++c)
         for (int i = cf_ptr[c]; i < cf_ptr[c + 1]; ++i) {
             int s = find(c, cf_nbr[i]);
@@ -431,7 +431,6 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
             V3 xN{d->cell_centre[3 * nb], d->cell_centre[3 * nb + 1], d->cell_centre[3 * nb + 2]};
             double w = vnorm({xf.x - xC.x, xf.y - xC.y, xf.z - xC.z}) / vnorm({xN.x - xC.x, xN.y - xC.y, xN.z - xC.z});
             cf_w[i] = w;
-            cf_omw[i] = 1.0 - w;
         }
     // every internal face is listed once by each of its two owners; the side's
     // nsign rides in the face's sign bit: ~face when -1
@@ -503,9 +502,7 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
     FVH_TRY(m->cf_face.upload(cf_face));
     FVH_TRY(m->cf_nbr.upload(cf_nbr));
     FVH_TRY(m->cf_slot.upload(cf_slot));
-    FVH_TRY(m->cf_sign.upload(cf_sign));
     FVH_TRY(m->cf_w.upload(cf_w));
-    FVH_TRY(m->cf_omw.upload(cf_omw));
     FVH_TRY(m->cf_fs.upload(cf_fs));
     FVH_TRY(m->own1.upload(own1));
     FVH_TRY(m->own2.upload(own2));
@@ -554,8 +551,7 @@ extern "C" int fvh_mesh_create(const fvh_mesh_desc *d, fvh_mesh **out) {
     v.n = n; v.nf = nf; v.nbf = nbf; v.nnz = nnz; v.ncf = ncf;
     v.rowptr = m->rowptr.p; v.col = m->col.p; v.diag = m->diag.p; v.tslot = m->tslot.p;
     v.cf_ptr = m->cf_ptr.p; v.cf_face = m->cf_face.p; v.cf_nbr = m->cf_nbr.p; v.cf_slot = m->cf_slot.p;
-    v.cf_sign = m->cf_sign.p; v.cf_w = m->cf_w.p; v.cf_omw = m->cf_omw.p;
-    v.nif = nif; v.cf_fs = m->cf_fs.p;
+    v.cf_w = m->cf_w.p; v.cf_fs = m->cf_fs.p;
     v.own1 = m->own1.p; v.own2 = m->own2.p; v.fw = m->fw.p; v.farea = m->farea.p; v.fdelta = m->fdelta.p;
     v.Sfx = m->Sfx.p; v.Sfy = m->Sfy.p; v.Sfz = m->Sfz.p; v.nx = m->nx.p; v.ny = m->ny.p; v.nz = m->nz.p;
     v.ex = m->ex.p; v.ey = m->ey.p; v.ez = m->ez.p;
