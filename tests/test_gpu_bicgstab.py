@@ -49,3 +49,56 @@ def test_bicgstab_against_the_oracle(mesh, precond):
             assert same_bits(phi.host(), want) and same_bits(st.rnorm, wst["rnorm"]), (bscale, itmax, rtol)
     finally:
         LIB().fvh_eqn_destroy(eq)
+
+
+@pytest.mark.parametrize("size", [(65, 33), (130, 64), (700, 400)])
+@pytest.mark.parametrize("precond", [L.PRECOND_DILU, L.PRECOND_ILU0, L.PRECOND_JACOBI, L.PRECOND_NONE])
+def test_fused_fp32_inner_solves(size, precond, monkeypatch):
+    """The FP32 solves inside the FP64 correction, with the products in the
+    sweeps' layout (or by band position) and in natural CSR rows: the same bits
+    where both apply one arithmetic (ILU(0)'s differs by walk).  Both reach
+    the FP64 solve's residual past the FP32 limit in a like number of iterations."""
+    got = {}
+    for sweep in ("band", "levels"):
+        if sweep == "levels":
+            monkeypatch.setenv("FVH_SWEEP", "levels")
+        else:
+            monkeypatch.delenv("FVH_SWEEP", raising=False)
+        mesh = F.channel(*size)
+        dm = mesh.device()
+        rp, ci = dm.pattern()
+        n = mesh.ncells
+        rng = np.random.default_rng(n)
+        rows = np.repeat(np.arange(n), np.diff(rp))
+        vals = np.where(rows == ci, 4.4 + rng.random(ci.size), -0.5 - 0.6 * rng.random(ci.size))
+        b, x = rng.standard_normal(n), 0.1 * rng.standard_normal(n)
+        defect = lambda y: np.linalg.norm(b - np.bincount(rows, vals * y[ci], n))  # noqa: E731
+        eq, nz, rhs = C.c_void_p(), C.c_void_p(), C.c_void_p()
+        L.check(LIB().fvh_eqn_create(dm.h, C.byref(eq)))
+        try:
+            L.check(LIB().fvh_eqn_arrays(eq, C.byref(nz), C.byref(rhs)))
+            L.check(LIB().fvh_memcpy(nz, vals.ctypes.data_as(C.c_void_p), vals.nbytes))
+            L.check(LIB().fvh_memcpy(rhs, b.ctypes.data_as(C.c_void_p), b.nbytes))
+            L.check(LIB().fvh_precond_set(eq, precond, None))
+            L.check(LIB().fvh_precond_update(eq))
+            its = {}
+            for precision, itmax, rtol in ((L.FP64, 200, 1e-9), (L.MIXED, 200, 1e-9), (L.MIXED, 1, 1e-4),
+                                           (L.MIXED, 2, 1e-4), (L.MIXED, 7, 1e-4)):
+                cfg = L.SolverCfg(solver=L.BICGSTAB, precond=precond, itmax=itmax, precision=precision,
+                                  convergence=0.0, relax=1.0, atol=0.0, rtol=rtol)
+                st, phi = L.Stats(), L.DeviceArray.from_host(x)
+                L.check(LIB().fvh_solve(eq, C.byref(cfg), phi.vp, C.byref(st)), "fvh_solve")
+                y = phi.host()
+                if itmax == 200:
+                    its[precision] = st.niter
+                    # the residual that stops FP64 is the preconditioned one
+                    assert defect(y) <= 1e-8 * defect(x), (sweep, precision, defect(y) / defect(x))
+                if precision == L.MIXED:
+                    got[sweep, itmax] = np.append(y, [st.niter, st.status, st.rnorm])
+            # a restart of the Krylov space at each of the few corrections
+            assert its[L.MIXED] <= 2 * its[L.FP64] + 4, its
+        finally:
+            LIB().fvh_eqn_destroy(eq)
+    if precond != L.PRECOND_ILU0:
+        for itmax in (200, 1, 2, 7):
+            assert same_bits(got["band", itmax], got["levels", itmax]), itmax

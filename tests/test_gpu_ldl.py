@@ -46,9 +46,9 @@ def _pressure_matrix(mesh, gamma, dm):
 @pytest.mark.parametrize("solves", ["ranges", "rows"])
 @pytest.mark.parametrize("name", REFERENCE_MESHES)
 def test_ldl_apply_against_the_oracle(ref_mesh, name, solves, monkeypatch):
-    """Both triangular-solve schedules: the range walk over the
-    nested-dissection leaves and separators (the default) and one wave per
-    row (FVH_LDL_RANGES=0)."""
+    """Both triangular-solve schedules: the block solves with the inverted
+    triangles of the nested-dissection leaves and separators (the default)
+    and one wave per row (FVH_LDL_RANGES=0)."""
     monkeypatch.setenv("FVH_LDL_RANGES", "1" if solves == "ranges" else "0")
     mesh = ref_mesh(name)
     dm = mesh.device()
