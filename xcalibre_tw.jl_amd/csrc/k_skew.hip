@@ -1490,7 +1490,10 @@ static int launch_sweeps_w(fvh_eqn *e, SkewSweep<T> &w, const KScal *ks) {
     return FVH_OK;
 }
 
-// FP32 ILU(0) applies the premultiplied records as DILU does
+// FP32 ILU(0) applies the premultiplied records as DILU does.  Its distance
+// from the FP64 apply, against that of the level walk's unpremultiplied
+// factors with a division (relative 2-norm): dominant 317 x 203 6.1e-8 / 6.8e-8,
+// Laplacian 6.3e-8 / 7.2e-8, upwinded rows 0.7-0.9e-7 / 1.4-1.9e-7.
 template <typename T, int W>
 static int launch_sweeps_k(fvh_eqn *e, SkewSweep<T> &w, const KScal *ks) {
     if constexpr (sizeof(T) == 8) {

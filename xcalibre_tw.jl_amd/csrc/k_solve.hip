@@ -302,7 +302,7 @@ int prepare32(fvh_eqn *e) {
     fvh_eqn *src = P->pmat ? P->pmat : P;
     switch (P->pkind) {
         case FVH_PRECOND_NONE: return FVH_OK;
-        case FVH_PRECOND_LDL: return FVH_OK;  // the factor keeps its own FP32 copy, made at set-up
+        case FVH_PRECOND_LDL: return FVH_OK;  // applied with the FP64 factor
         case FVH_PRECOND_JACOBI:
         case FVH_PRECOND_NORMDIAG: {
             if (P->p32a.n != (size_t)n) FVH_TRY(P->p32a.alloc(n));
