@@ -10,11 +10,12 @@
 //   -> scheme_source! terms -> sources
 //   -> boundary conditions (BC tuple order, then patch face order, then terms)
 //   -> implicit relaxation -> setReference!.
-// Bound by HBM.  Each face is read by both its cells, the second time mostly
-// from a cache (its cells are near each other), and its coefficient is formed
-// twice.  That moves 56 % of the bytes of a face pass that hands each side's
-// diagonal terms to a cell pass through memory (2000 x 1000 quads, two face
-// terms: 178 us; this pass: 101 us).
+// Bound by HBM.  Each face is read by both its cells and its coefficient is
+// formed twice; three quarters of the second reads hit L2.  2000 x 1000 quads,
+// two face terms, traffic by counters: 271 MB read (240 with each face once)
+// and 140 MB written (96 MB of values: a row's stores leave one by one), 101
+// us.  A face pass that hands each side's diagonal terms to a cell pass through
+// memory moves 807 MB in 178-206 us.
 #include "fvh_eqn.h"
 
 namespace fvh {
