@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <limits>
+#include <type_traits>
 
 #include "fvh_eqn.h"
 #include "k_band.h"
@@ -185,7 +186,7 @@ static int ilu_setup(fvh_mesh *m) {
 
 // ILU(0) runs on the pipelined band sweeps on a single full rectangle (250 x
 // 125: 65 us an apply, against 771 us on the one-work-group level walk, which
-// keeps the other meshes).
+// keeps the other meshes; 8 x 8: 17 / 18; a handful of cells, 3 x 2: 16 / 5).
 static bool ilu_skew(const fvh_mesh *m) { return !m->cases && band_path(m) && skew_active(m); }
 
 int precond_update(fvh_eqn *eq) {
@@ -714,6 +715,10 @@ struct BandRows {
         return band_ax_at(n, nx, mask, C, xat, i);
     }
 };
+// No product: the vector update alone (the system's own SpMV follows)
+struct NoRows {
+    static constexpr bool kXcd = false;
+};
 template <typename V>
 struct CsrRows {
     static constexpr bool kXcd = false;
@@ -745,8 +750,8 @@ static int launch_rows(fvh_eqn *e, L launch) {
 // its own and each product a gather and a scatter (20): a block forms the
 // scalar it needs from the partial sums itself (as CG's do), the vector
 // updates p' and s run inside the products that read them (a neighbour's value
-// is formed again by the owner's expression), x takes both its updates in one
-// pass.  us per iteration with the solve's set-up, one launch each / fused,
+// is formed again by the owner's expression; eleven launches past kBiInside
+// rows, where they don't), x takes both its updates in one pass.  us per iteration with the solve's set-up, one launch each / fused,
 // DILU: FP64 40x40 90/63, 64x63 100/68, 130x90 126/94, 250x125 156/123,
 // 1000x1000 642/625; FP32 40x40 132/95, 130x90 152/108, 1000x1000 452/420.
 // At 1M rows in FP64 k_bi_s takes 47-55 us, most of it the scatter into the
@@ -821,7 +826,7 @@ __global__ void __launch_bounds__(kBlock)
     const auto pnew = [=](int j) -> T { return bi_p<T>(r[j], p[j], v[j], om, be); };
     for (int i = row_block<Ax>() * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         pn[i] = pnew(i);
-        out.put(n, i, ax(pnew, i));
+        if constexpr (!std::is_same_v<Ax, NoRows>) out.put(n, i, ax(pnew, i));
     }
 }
 // alpha from the partial sums of b.v, s = r - alpha v and the product A s
@@ -841,7 +846,7 @@ __global__ void __launch_bounds__(kBlock)
     const auto snew = [=](int j) -> T { return D(r[j]) + (-al) * D(v[j]); };
     for (int i = row_block<Ax>() * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         s[i] = snew(i);
-        out.put(n, i, ax(snew, i));
+        if constexpr (!std::is_same_v<Ax, NoRows>) out.put(n, i, ax(snew, i));
     }
 }
 // omega from the partial sums of t.s and t.t, both updates of x, r = s - omega
@@ -874,6 +879,23 @@ __global__ void __launch_bounds__(kWide)
         sp[1][j] = rr;
     }
     chunk_reduce_staged<2>(sp, pout, nch, blockIdx.x);
+}
+
+// Rows up to which the vector updates run inside the products: past it a
+// neighbour's p' and s, formed again from two or three vectors, come from
+// memory.  us an iteration, Jacobi, inside / apart (and in one launch a scalar,
+// a gather and a scatter): FP64 CSR quads 490k rows 56/57 (64), 1M 83/80 (87),
+// 1.5M 122/115 (117), 3M 240/222 (228), 4.5M 358/326 (332); FP32 490k 46/55
+// (62), 1M 63/66 (74), 3M 142/132 (138).  Into the sweeps' layout (grids up to
+// about 2M rows) they always go inside: DILU on 1500 x 1000 FP64 885/873 (889),
+// FP32 427/449 (469).
+constexpr int kBiInside = 1 << 20;
+template <typename T, class L>
+static int launch_rows_if(fvh_eqn *e, bool product, L launch) {
+    if (product) return launch_rows<T>(e, launch);
+    launch(NoRows{});
+    HIP_TRY(hipGetLastError());
+    return FVH_OK;
 }
 
 template <typename T>
@@ -940,6 +962,7 @@ static int bicgstab(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats
         out = RhsOut<T>{static_cast<T *>(rt.dst), rt.map, rt.stride, static_cast<T *>(rt.hand), rt.nhand, rt.HS, rt.sent};
     }
     const int nch = nchunks(n);
+    const bool fuse = qmap || n <= kBiInside;
     first_batch(e);
     while (!w.h_ks->done && enq < itmax) {
         int nb = std::min(next_batch(enq), itmax - enq);
@@ -947,12 +970,13 @@ static int bicgstab(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats
             const T *nat = nullptr;  // the product in natural rows (its gather runs in the apply)
             if (it > 0) {
                 T *pn = t;  // t is free until the second apply
-                FVH_TRY(launch_rows<T>(e, [&](auto ax) {
+                FVH_TRY(launch_rows_if<T>(e, fuse, [&](auto ax) {
                     hipLaunchKernelGGL(k_bi_p, fused_grid(n), dim3(kBlock), 0, stream(), n, part2, nch, ks, itmax, r,
                                        p, v, pn, out, ax);
                 }));
                 std::swap(p, t);
-            } else {
+            }
+            if (it == 0 || !fuse) {
                 FVH_TRY(sys_spmv(S, p, q, ks));
                 nat = q;
             }
@@ -965,12 +989,13 @@ static int bicgstab(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats
                     if (qmap) v[i] = y.a;
                     a[0] = D(y.b) * D(y.a);
                 }));
-            FVH_TRY(launch_rows<T>(e, [&](auto ax) {
+            FVH_TRY(launch_rows_if<T>(e, fuse, [&](auto ax) {
                 hipLaunchKernelGGL(k_bi_s, fused_grid(n), dim3(kBlock), 0, stream(), n, part, nch, ks, r, v, s, out, ax);
             }));
+            if (!fuse) FVH_TRY(sys_spmv(S, s, q, ks));
             const T *tq = nullptr;
             T *tt = t;
-            if (qmap) FVH_TRY(sys_precond_quads(S, nullptr, ks, &tq));
+            if (qmap) FVH_TRY(sys_precond_quads(S, fuse ? nullptr : q, ks, &tq));
             else FVH_TRY(sys_precond(S, t, q, ks));
             FVH_TRY(mapred_wide<2>(
                 n, ks, part, [=] __device__(int i) { return Pair<T>{qmap ? tq[qmap[i]] : tt[i], s[i]}; },
@@ -1290,8 +1315,19 @@ static int gmres(const Sys<T> &S, const fvh_solver_cfg &cfg, T *xu, fvh_stats *s
             FVH_TRY(mapred_wide<1>(n, ks, pin, [=] __device__(int j) { return Pair<T>{V[j], q[j]}; },
                                    [=] __device__(int, const Pair<T> &v, double(&a)[1]) { a[0] = D(v.a) * D(v.b); }));
             for (int i = 0; i < k; ++i) {
+                double *Ri = R + nr + i;
+                const T *Vi = V + (size_t)i * ld, *Vn = i + 1 < k ? Vi + ld : nullptr;
+                if (n > kLatencyRows) {
+                    FVH_TRY(finalize<1>(n, pin, ks, true, [=] __device__(KScal *, double(&d)[1]) { *Ri = d[0]; }));
+                    FVH_TRY(mapred<1>(n, ks, pin, [=] __device__(int j, double(&a)[1]) {
+                        const T qj = D(q[j]) + (-(*Ri)) * D(Vi[j]);
+                        q[j] = qj;
+                        a[0] = a[0] + (Vn ? D(Vn[j]) : D(qj)) * D(qj);
+                    }));
+                    continue;
+                }
                 hipLaunchKernelGGL((k_mgs<T>), dim3(nchunks(n)), dim3(kWide), 0, stream(), n, pin, pout, nchunks(n), ks,
-                                   R + nr + i, V + (size_t)i * ld, i + 1 < k ? V + (size_t)(i + 1) * ld : nullptr, q);
+                                   Ri, Vi, Vn, q);
                 HIP_TRY(hipGetLastError());
                 std::swap(pin, pout);
             }

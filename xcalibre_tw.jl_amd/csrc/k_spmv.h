@@ -139,6 +139,16 @@ __device__ inline void chunk_reduce_staged(double (&p)[NV][kChunk], double *__re
     }
 }
 
+// Rows up to which a vector pass is bound by latency rather than by memory
+// (three FP64 vectors then still fit the L2s and the Infinity Cache beside the
+// matrix): one kWide block per chunk, all loads in flight, and sums formed by
+// every block.  Past it k_mapred's eight rows a thread, whose blocks hold no
+// LDS and meet at no barrier between their loads, and a launch for each sum move
+// more: GMRES + Jacobi, us an iteration of ten, below / above forms, FP64 quads
+// 1M rows 87/110, 2M 169/179, 2.5M 221/213, 3.6M 309/274; FP32 2M 88/91, 2.5M
+// 107/102, 3.6M 158/138.
+constexpr int64_t kLatencyRows = 1 << 21;
+
 // Elementwise work + partial sums over the canonical chunks, one block of
 // kWide threads per chunk: a thread's rows are loaded (load(i)) before the
 // first of their results is written (op(i, v, a) sets the row's terms a), so
@@ -170,6 +180,13 @@ __global__ void __launch_bounds__(kWide) k_mapred_wide(int n, const KScal *ks, d
 template <int NV, class Ld, class Op>
 inline int mapred_wide(int64_t n, const KScal *ks, double *part, Ld load, Op op) {
     const int nch = nchunks(n);
+    if (n > kLatencyRows)
+        return mapred<NV>(n, ks, part, [=] __device__(int i, double(&a)[NV]) {
+            double t[NV];
+            op(i, load(i), t);
+#pragma unroll
+            for (int q = 0; q < NV; ++q) a[q] = a[q] + t[q];
+        });
     hipLaunchKernelGGL((k_mapred_wide<NV, Ld, Op>), dim3(nch > 0 ? nch : 1), dim3(kWide), 0, stream(), (int)n, ks, part,
                        nch, load, op);
     HIP_TRY(hipGetLastError());
