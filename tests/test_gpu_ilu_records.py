@@ -108,7 +108,10 @@ def test_dilu_and_ilu0_in_turn_on_one_equation(nx, ny):
                 assert LIB().fvh_precond_apply_f32(eq.h, fy.vp, fx.vp) == L.FVH_ERR_ARG
             eq.update(mats[second])
             assert same_bits(eq.apply(x), want[second][0]) and same_bits(eq.apply(x, True), want[second][1])
-            eq.set(first)  # as updated before
-            assert same_bits(eq.apply(x), want[first][0]) and same_bits(eq.apply(x, True), want[first][1])
-            eq.set(L.PRECOND_DILU)
-            assert same_bits(eq.dinv(), want[L.PRECOND_DILU][2])
+            if second == L.PRECOND_DILU:
+                assert same_bits(eq.dinv(), want[L.PRECOND_DILU][2])
+            if min(nx, ny) > 1:  # as updated before (elsewhere a set-up allocates anew)
+                eq.set(first)
+                assert same_bits(eq.apply(x), want[first][0]) and same_bits(eq.apply(x, True), want[first][1])
+                eq.set(L.PRECOND_DILU)
+                assert same_bits(eq.dinv(), want[L.PRECOND_DILU][2])
